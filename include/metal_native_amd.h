@@ -236,7 +236,7 @@ MQ_API int mq_read_probe(const void* p, int64_t bytes, void* sink, void* stream)
 /* Kernel-path override and layout knobs for tests and tuning (no reference
  * counterpart).  Keys: "force_path" (0 automatic, 2 the prefill GEMM family,
  * 3 generic, 6 split-K decode GEMV, 7 row-block decode GEMV, 12 register-
- * streamed decode GEMV: int4, 3 <= M <= 16), "gemv_steps"
+ * streamed decode GEMV: int4, 3 <= M <= 16, 13 many-row GEMM), "gemv_steps"
  * (K steps per wavefront of the split-K GEMV, 1..8, 0 automatic),
  * "gemv_tiles_per_wg" (row tiles per workgroup: 1, 2 or 4, 0 automatic),
  * "gemm_impl" (prefill GEMM kernel: 0 automatic -- the register-dequant
@@ -244,7 +244,9 @@ MQ_API int mq_read_probe(const void* p, int64_t bytes, void* sink, void* stream)
  * where its tiles fill the GPU, else the register-operand 32x32x16 kernel
  * where it takes the shape --, 1 always the 16x16x32 tiled kernel, 2 the
  * register-dequant GEMM wherever it takes the shape; all compute the same
- * contract), "gemm_split" (1, the default: the 32x32x16 kernel splits
+ * contract), "gemm_rows" (rows per tile of the many-row GEMM: 128 or 256, 0 automatic)
+ * and "gemm_parts" (its K parts, 1..16, 0 automatic), both read when
+ * force_path is 13, "gemm_split" (1, the default: the 32x32x16 kernels split
  * K over several workgroups per output tile where its tiles would leave CUs
  * idle, summing the parts in a fixed order; 0: one workgroup per tile).  A forced path that cannot take the shape falls back
  * to the automatic choice.  Returns MQ_INVALID_ARGUMENT for an unknown key or
@@ -256,7 +258,7 @@ MQ_API int mq_set_option(const char* key, int64_t value);
  * generic, 4 vecmat [K,N], 6 split-K decode GEMV, 7 row-block decode GEMV, 8
  * 32x32x16 prefill GEMM, 9 fp32 vecmat, 10 32x32x16 prefill GEMM with K split
  * over workgroups, 11 register-dequant 16x16x32 prefill GEMM, 12
- * register-streamed decode GEMV. */
+ * register-streamed decode GEMV, 13 many-row GEMM. */
 MQ_API int mq_last_path(void);
 
 MQ_API const char* mq_last_error(void);

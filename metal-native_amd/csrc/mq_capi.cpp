@@ -56,16 +56,22 @@ int num_cus_current() {
 // over workgroups) or PATH_TILED (the 16x16x32 fallback).
 enum Path {
   PATH_AUTO = 0, PATH_TILED = 2, PATH_GENERIC = 3, PATH_VECMAT_KN = 4, PATH_DECODE = 6, PATH_ROWS = 7,
-  PATH_GEMMW = 8, PATH_VECMAT32 = 9, PATH_GEMMW_SPLIT = 10, PATH_GEMM16 = 11, PATH_RSTREAM = 12
+  PATH_GEMMW = 8, PATH_VECMAT32 = 9, PATH_GEMMW_SPLIT = 10, PATH_GEMM16 = 11, PATH_RSTREAM = 12,
+  PATH_GEMMN = 13
 };
 // prefill GEMM choice (gemm_impl): 0 automatic (the register-dequant GEMM where
 // its tiles fill the GPU, else the register-operand 32x32x16 kernel where it
 // takes the shape), 1 always the 16x16x32 tiled kernel, 2 the register-dequant
 // GEMM wherever it takes the shape
 std::atomic<int> g_gemm_impl{0};
-// gemm_split: 1 lets the 32x32x16 kernel split K over workgroups where its
+// gemm_split: 1 lets the 32x32x16 kernels split K over workgroups where their
 // tiles leave CUs idle, 0 keeps one workgroup per tile
 std::atomic<int> g_gemm_split{1};
+
+// gemm_rows: rows per tile of the many-row GEMM (128 or 256), 0 automatic
+std::atomic<int> g_gemm_rows{0};
+// gemm_parts: K parts of the many-row GEMM (1..16), 0 automatic
+std::atomic<int> g_gemm_parts{0};
 
 mq::GemvTuning gemv_tuning() {
   mq::GemvTuning t;
@@ -141,6 +147,31 @@ bool gemm16_auto(const mq::LinearArgs& a) {
   return 4 * (int64_t)mq::gemm16_workgroups(a) >= 3 * (int64_t)num_cus_current() && 4 * (int64_t)a.M >= 3 * mpad;
 }
 
+// The many-row GEMM (mq_gemmn.hip), automatically: where its launch-time
+// model is at least 7 % below that of the kernel the shape would take
+// otherwise, and that one is 25 us or more (below, the models' errors exceed
+// the gain).  On 208 measured shapes (M = 32..4096) the choice is the faster
+// kernel or within 6 % of it on all but 5, e.g. M = 4096, K = 3584, N = 37888
+// int4 SwiGLU: 1.05 ms against 2.51; M = 777, K = 18944, N = 3584: 134 us
+// against 278; M = 512, K = 3072, N = 5120 stays with the 16x16x32 GEMM (23
+// against 35 us).
+mq::GemmnPlan gemmn_auto(const mq::LinearArgs& a, bool allow_split) {
+  const int cus = num_cus_current();
+  allow_split = allow_split && g_gemm_split.load() != 0;
+  mq::GemmnPlan none{};
+  if (a.M <= 16 || g_gemm_impl.load() != 0 || !mq::gemmn_supported(a)) return none;
+  double other = 1e30;   // the 16x16x32 kernel's fallback: always slower
+  if (gemm16_auto(a)) {
+    if (mq::gemm16_rows_per_tile(a) != 128) return none;   // 64-row SwiGLU tiles: made for M <= 64
+    other = mq::gemm16_estimate(a, cus);
+  } else if (mq::gemmw_supported(a, cus)) {
+    other = mq::gemmw_estimate(a, cus, allow_split);
+  }
+  if (other < 25.0) return none;
+  const mq::GemmnPlan p = mq::gemmn_plan(a, cus, allow_split);
+  return p.ok && p.us < 0.93 * other ? p : none;
+}
+
 // Short weight rows over many of them, M <= 4: the split-K GEMV, whose
 // start-up is shorter than the row-block kernel's staging of all of K.
 // Measured on 108 shapes (M = 1, 2, 4; K = 512..3584; N = 896, 4864, 14336;
@@ -160,6 +191,7 @@ int choose_path(const mq::LinearArgs& a, bool noalloc) {
   if (forced == PATH_RSTREAM && mq::rstream_plan(a, num_cus_current()).ok) return PATH_RSTREAM;
   if (forced == PATH_DECODE && decode_ok(a)) return PATH_DECODE;
   if (forced == PATH_TILED && prefill_ok(a)) return PATH_TILED;
+  if (forced == PATH_GEMMN && mq::gemmn_supported(a)) return PATH_GEMMN;
   if (forced == PATH_GENERIC) return PATH_GENERIC;
   // automatic choice: the row-block kernel up to M = 4; for M = 5..16 only
   // where the activations fit in LDS whole (its K parts measured slower than
@@ -188,6 +220,7 @@ int choose_path(const mq::LinearArgs& a, bool noalloc) {
       mq::gemmw_supported(a, num_cus_current()) && mq::gemmw_ws_bytes(a, num_cus_current(), true) > 0)
     return PATH_TILED;
   if (decode_ok(a)) return PATH_DECODE;
+  if (gemmn_auto(a, !noalloc).ok) return PATH_GEMMN;
   if (prefill_ok(a)) return PATH_TILED;
   return PATH_GENERIC;
 }
@@ -213,10 +246,29 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
       path = decode_ok(a) ? PATH_DECODE : PATH_GENERIC;
     }
   }
+  if (path == PATH_GEMMN) {
+    const int rows = g_gemm_rows.load(), parts = g_gemm_parts.load();
+    auto planned = [&](bool split) {
+      return g_force_path.load() == PATH_GEMMN ? mq::gemmn_plan(a, num_cus_current(), split, rows / 32, split ? parts : 1)
+                                               : gemmn_auto(a, split);
+    };
+    mq::GemmnPlan pl = planned(!noalloc);
+    void* ws = nullptr;
+    e = workspace_for(s, pl.ws_bytes, &ws);
+    if (e == hipErrorStreamCaptureUnsupported) {
+      // under capture with a workspace too small for this shape: the choice
+      // among the kernels that need none
+      e = hipSuccess;
+      pl = planned(false);
+      if (!pl.ok) path = PATH_TILED;
+    }
+    if (e != hipSuccess) return hip_fail(e, "dequant_matmul: workspace allocation failed");
+    if (pl.ok) e = mq::gemmn_launch(a, pl, ws, s);
+  }
   if (path == PATH_RSTREAM) {
     const mq::RsPlan pl = mq::rstream_plan(a, num_cus_current());
     e = pl.ok ? mq::rstream_launch(a, pl, s) : hipErrorInvalidValue;
-  } else if (path == PATH_ROWS) {
+  } else if (path == PATH_ROWS || path == PATH_GEMMN) {
   } else if (path == PATH_DECODE) {
     const mq::GemvPlan pl = mq::gemv_plan(a, num_cus_current(), gemv_tuning());
     void* ws = nullptr;
@@ -647,8 +699,8 @@ MQ_API int mq_set_option(const char* key, int64_t value) {
   if (!key) return fail(MQ_INVALID_ARGUMENT, "set_option: null key");
   if (std::strcmp(key, "force_path") == 0) {
     if (value != PATH_AUTO && value != PATH_TILED && value != PATH_GENERIC && value != PATH_DECODE &&
-        value != PATH_ROWS && value != PATH_RSTREAM)
-      return fail(MQ_INVALID_ARGUMENT, "set_option: force_path must be 0, 2, 3, 6, 7 or 12");
+        value != PATH_ROWS && value != PATH_RSTREAM && value != PATH_GEMMN)
+      return fail(MQ_INVALID_ARGUMENT, "set_option: force_path must be 0, 2, 3, 6, 7, 12 or 13");
     g_force_path.store((int)value);
     return MQ_SUCCESS;
   }
@@ -661,6 +713,17 @@ MQ_API int mq_set_option(const char* key, int64_t value) {
   if (std::strcmp(key, "gemm_split") == 0) {
     if (value != 0 && value != 1) return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_split must be 0 or 1");
     g_gemm_split.store((int)value);
+    return MQ_SUCCESS;
+  }
+  if (std::strcmp(key, "gemm_rows") == 0) {
+    if (value != 0 && value != 128 && value != 256)
+      return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_rows must be 0, 128 or 256");
+    g_gemm_rows.store((int)value);
+    return MQ_SUCCESS;
+  }
+  if (std::strcmp(key, "gemm_parts") == 0) {
+    if (value < 0 || value > 16) return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_parts must be 0..16");
+    g_gemm_parts.store((int)value);
     return MQ_SUCCESS;
   }
   if (std::strcmp(key, "gemv_steps") == 0) {

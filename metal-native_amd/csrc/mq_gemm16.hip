@@ -675,6 +675,16 @@ int gemm16_workgroups(const LinearArgs& a) {
   return ((a.M + 16 * sh.mbk - 1) / (16 * sh.mbk)) * ((nout + bno - 1) / bno);
 }
 
+// Fitted to measured launches of the 128 x 80 tiles (M = 192..4096, K =
+// 896..18944; 13 % rms): 5.4 us per round of workgroups and 1.32 us per
+// K-tile of a wave, 12 % more per further round (up to 6) as the clock drops
+// under the load.
+double gemm16_estimate(const LinearArgs& a, int cus) {
+  const double r = (double)gemm16_workgroups(a) / cus;
+  const double per = 5.4 + a.K / 256.0 * (1.32 + 0.116 * std::max(0.0, std::min(r, 6.0) - 1.0));
+  return 4.3 + (r < 3.0 ? std::ceil(r) : r + 0.4) * per;
+}
+
 hipError_t gemm16_launch(const LinearArgs& a, hipStream_t s, uint64_t* trace) {
   if (!shape_ok(a)) return hipErrorInvalidValue;
   const G16Shape sh = pick(a);

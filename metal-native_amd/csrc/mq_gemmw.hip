@@ -556,6 +556,20 @@ bool sz_table_fits(const LinearArgs& a, int BN) {
 // VALU, texture-unit requests and the tile's weight bytes at its share of
 // ~6 TB/s; the launch takes ceil(tiles / CUs) tile times (one workgroup per
 // CU).
+// Launch time (us) of MB x NB tiles with KP K parts each: fitted to 290
+// measured launches (int4, M = 17..128, K = 2048..18944): per-wave K-tiles
+// times the tile's MFMA, dequant and activation work, rounds of workgroups
+// over the CUs, and for K parts a fixed cost plus the last arriver's reads of
+// the parts.  (14 % rms over a further 80 launches up to M = 4096.)
+double launch_us(int K, int MB, int NB, int64_t tiles, int KP, int cus) {
+  const double per = std::ceil(K / 64.0) / KP / 4.0;
+  const double rounds = std::ceil((double)(tiles * KP) / cus);
+  const double rp = rounds * per;
+  const double sp = KP > 1 ? 1.0 : 0.0;
+  return -5.09 + rp * (0.1544 + 0.1768 * MB * NB + 0.0858 * NB - 0.1602 * MB) + sp * (2.78 + 0.1575 * KP * MB * NB) +
+         11.39 * rounds;
+}
+
 WPlan plan(const LinearArgs& a, int cus, bool allow_split) {
   WPlan best{};
   best.ok = false;
@@ -602,20 +616,10 @@ WPlan plan(const LinearArgs& a, int cus, bool allow_split) {
   }
   // K split over workgroups, where the tiles above leave at least half the
   // CUs idle: candidates of 2 weight blocks (wider tiles measured slower at
-  // these shapes) and 1, 2 or 4 A blocks, with 1..8 K parts of at least 8 K-tiles each, priced by a
-  // launch-time model fitted to 290 measured launches (int4, M = 17..128, K
-  // = 2048..18944): per-wave K-tiles times the tile's MFMA, dequant and
-  // activation work, rounds of workgroups over the CUs, and for K parts a
-  // fixed cost plus the last arriver's reads of the parts.
+  // these shapes) and 1, 2 or 4 A blocks, with 1..8 K parts of at least 8
+  // K-tiles each, priced by launch_us.
   if (best.ok && allow_split && (int64_t)best.nbm * best.nbn * 2 <= cus) {
-    auto fitted = [&](int MB, int NB, int64_t tiles, int KP) {
-      const double per = kt / KP / 4.0;
-      const double rounds = std::ceil((double)(tiles * KP) / cus);
-      const double rp = rounds * per;
-      const double sp = KP > 1 ? 1.0 : 0.0;
-      return -5.09 + rp * (0.1544 + 0.1768 * MB * NB + 0.0858 * NB - 0.1602 * MB) + sp * (2.78 + 0.1575 * KP * MB * NB) +
-             11.39 * rounds;
-    };
+    auto fitted = [&](int MB, int NB, int64_t tiles, int KP) { return launch_us(a.K, MB, NB, tiles, KP, cus); };
     double fbest = fitted(best.MB, best.NB, (int64_t)best.nbm * best.nbn, 1);
     const int NB = 2;
     // one A block per tile where M <= 32 (12-17 % faster than two at M = 16..32)
@@ -701,6 +705,11 @@ bool gemmw_supported(const LinearArgs& a, int cus) {
 }
 
 size_t gemmw_ws_bytes(const LinearArgs& a, int cus, bool allow_split) { return plan(a, cus, allow_split).ws_bytes; }
+
+double gemmw_estimate(const LinearArgs& a, int cus, bool allow_split) {
+  const WPlan p = plan(a, cus, allow_split);
+  return p.ok ? launch_us(a.K, p.MB, p.NB, (int64_t)p.nbm * p.nbn, p.KP, cus) : 0.0;
+}
 
 hipError_t gemmw_launch(const LinearArgs& a, int cus, void* ws, hipStream_t s, bool allow_split) {
   const WPlan pl = plan(a, cus, allow_split);

@@ -112,6 +112,8 @@ hipError_t rstream_launch(const LinearArgs& a, const RsPlan& p, hipStream_t s);
 // that every launch leaves at zero, then the partial sums).
 bool gemmw_supported(const LinearArgs& a, int num_cus);
 size_t gemmw_ws_bytes(const LinearArgs& a, int num_cus, bool allow_split);
+// estimated launch time (us) of the plan, 0 when there is none
+double gemmw_estimate(const LinearArgs& a, int num_cus, bool allow_split);
 hipError_t gemmw_launch(const LinearArgs& a, int num_cus, void* ws, hipStream_t s, bool allow_split);
 
 // 128-row int4 GEMM (16x16x32 MFMA, one workgroup per 128 x 80 tile, no
@@ -119,7 +121,22 @@ hipError_t gemmw_launch(const LinearArgs& a, int num_cus, void* ws, hipStream_t 
 bool gemm16_supported(const LinearArgs& a);
 int gemm16_workgroups(const LinearArgs& a);
 int gemm16_rows_per_tile(const LinearArgs& a);
+double gemm16_estimate(const LinearArgs& a, int num_cus);   // launch time (us)
 hipError_t gemm16_launch(const LinearArgs& a, hipStream_t s, uint64_t* trace);
+
+// GEMM for many rows (32x32x16 MFMA, waves side by side along N, shared
+// activation tiles, no workspace): 32 * mb rows per tile, mb = 4 or 8.
+bool gemmn_supported(const LinearArgs& a);
+// K may be split over KP workgroups per tile, whose fp32 sums (ws_bytes, need
+// not be cleared) a second kernel adds up.
+struct GemmnPlan {
+  int mb, KP, ktp;   // 32-row blocks per tile, K parts, 64-k tiles per part
+  size_t ws_bytes;
+  double us;         // estimated time of the launch
+  bool ok;
+};
+GemmnPlan gemmn_plan(const LinearArgs& a, int num_cus, bool allow_split, int mb = 0, int kp = 0);
+hipError_t gemmn_launch(const LinearArgs& a, const GemmnPlan& p, void* ws, hipStream_t s);
 
 // 16x16x32 MFMA GEMM, K steps of 32 (fallback for shapes the GEMM above does not take).
 bool tiled_supported(const LinearArgs& a);

@@ -11,7 +11,8 @@ GEMV/GEMM epilogue (``dequant_matmul(..., epilogue="bias")``).  The library
 picks the kernel by the number of rows: the row-block GEMV for M <= 4, and
 up to M = 16 where the activations fit in LDS; for int4 at M = 5..16 the
 register-streamed GEMV where its plan takes the shape; the split-K GEMV for
-short rows and what the others decline; the MFMA GEMM beyond M = 16.  Built from fp16 weights (``from_float``, quantized on the GPU by
+short rows and what the others decline; beyond M = 16 one of the MFMA GEMMs,
+by the number of output tiles.  Built from fp16 weights (``from_float``, quantized on the GPU by
 ``quantize``) or from a ``QuantizedWeight`` (a loaded or converted
 checkpoint, ``from_quantized``).
 """

@@ -1,0 +1,231 @@
+"""The many-row prefill GEMM (mq_gemmn.hip) against the oracle: tile edges and
+remainders, K tails, groups, epilogues, strided operands, K parts, special
+scales, and the routing that chooses it."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import mq_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+TOL_ABS = 1e-2   # the contract's bound on a matmul output
+TOL_REL = 1e-3
+
+
+@pytest.fixture(scope="module")
+def mn(gpu):
+    import metal_native
+
+    yield metal_native
+    for key in ("force_path", "gemm_rows", "gemm_parts"):
+        metal_native.set_option(key, 0)
+
+
+def dev(x, gpu):
+    return torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+
+
+class forced:
+    """The kernel with `rows` per tile and `parts` K parts, whatever the planner would take."""
+
+    def __init__(self, mn, rows, parts):
+        self.mn, self.opts = mn, {"force_path": 13, "gemm_rows": rows, "gemm_parts": parts}
+
+    def __enter__(self):
+        for k, v in self.opts.items():
+            self.mn.set_option(k, v)
+
+    def __exit__(self, *exc):
+        for k in self.opts:
+            self.mn.set_option(k, 0)
+
+
+def problem(M, K, N, g, qt, seed):
+    if qt == "int4":
+        x, wp, s, z = O.make_int4_problem(M, K, N, g, seed=seed)
+        return x, wp, s, z, g, O.matmul_f32acc(x, O.dequant_int4(wp, s, z, K, g))
+    x, wp, s, z, g = O.make_int8_problem(M, K, N, seed=seed, g=g or None)
+    z = np.random.default_rng(3).uniform(-0.01, 0.01, s.shape).astype(np.float16)
+    return x, wp, s, z, g, O.matmul_f32acc(x, O.dequant_int8(wp, s, z, K, g))
+
+
+def silu(v):
+    with np.errstate(over="ignore"):
+        return v / (1.0 + np.exp(-v))
+
+
+def expected(acc, epi, bias, res):
+    """(reference in float64, extra tolerance): SiLU's is its change across
+    one fp16 (SwiGLU: of gate and up) or fp32 rounding of its argument."""
+    v = acc.astype(np.float64)
+    extra = 0.0
+    if epi == "swiglu":
+        F = v.shape[1] // 2
+        gate, up = (v[:, i * F:(i + 1) * F].astype(np.float16).astype(np.float64) for i in range(2))
+        ulp = np.spacing(np.maximum(np.abs(gate), np.abs(up)).astype(np.float16)).astype(np.float64)
+        return silu(gate) * up, ulp * (1.1 * np.abs(up) + np.abs(silu(gate)) + 1.1 * ulp)
+    if bias is not None:
+        v = v + bias.astype(np.float64)[None, :]
+    if res is not None:
+        v = v + res.astype(np.float64)
+    if epi == "bias_relu":
+        v = np.maximum(v, 0.0)
+    if epi == "bias_silu":
+        v = silu(v)
+    return v, extra
+
+
+def check(y, acc, epi=None, bias=None, res=None, what=""):
+    ref, extra = expected(acc, epi, bias, res)
+    err = np.abs(y.astype(np.float64) - ref)
+    bad = ~(err <= TOL_ABS + TOL_REL * np.abs(ref) + extra)
+    assert not bad.any(), f"{what}: {bad.sum()} of {bad.size} outside tolerance; max abs err {np.nanmax(err):.3g}"
+
+
+def epilogue_args(epi, M, N, gpu):
+    rng = np.random.default_rng(M + N)
+    if epi and epi.startswith("bias"):
+        b = rng.standard_normal(N).astype(np.float16)
+        return {"epilogue": epi, "bias": dev(b, gpu)}, b, None
+    if epi == "residual":
+        r = rng.standard_normal((M, N)).astype(np.float16)
+        return {"epilogue": epi, "residual": dev(r, gpu)}, None, r
+    return ({"epilogue": epi} if epi else {}), None, None
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("parts", [1, 3])
+@pytest.mark.parametrize("M,K,N,g,qt,epi", [
+    (1, 64, 2, 32, "int4", None),              # one K-tile, one row
+    (127, 256, 256, 64, "int4", "bias"),       # four K-tiles, last row short of a tile
+    (129, 320, 257, 32, "int4", None),         # five K-tiles, odd N: 2-byte stores
+    (257, 416, 520, 32, "int4", "residual"),   # K ends inside a K-tile
+    (200, 896, 1030, 128, "int4", "bias_silu"),
+    (64, 1184, 516, 32, "int4", "swiglu"),     # up rows of a partial tile; K tail
+    (255, 384, 254, 0, "int8", None),          # per-channel
+    (130, 160, 300, 32, "int8", "bias_relu"),
+    (300, 512, 770, 64, "int8", "swiglu"),
+    (31, 96, 96, 32, "int8", "residual"),
+])
+def test_against_oracle(mn, gpu, rows, parts, M, K, N, g, qt, epi):
+    x, wp, s, z, g, acc = problem(M, K, N, g, qt, seed=M + K + N)
+    kw, b, r = epilogue_args(epi, M, N, gpu)
+    with forced(mn, rows, parts):
+        run = lambda: mn.dequant_matmul(dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, qt, **kw)
+        y = run()
+        assert mn.last_path() == "gemmn"
+        check(y.cpu().numpy(), acc, epi, b, r, f"rows={rows} parts={parts}")
+        assert torch.equal(run(), y)   # a fixed summation order
+
+
+@pytest.mark.parametrize("rows,parts", [(128, 1), (256, 1), (128, 2)])
+@pytest.mark.parametrize("pad", [8, 3])
+def test_strided_operands(mn, gpu, rows, parts, pad):
+    """Activations, weights and output as column ranges of wider tensors, the
+    residual in place: nothing is read or written outside them."""
+    M, K, N, g = 150, 416, 266, 32
+    x, wp, s, z, g, acc = problem(M, K, N, g, "int4", seed=9)
+    xs = torch.full((M, K + 8), float("nan"), dtype=torch.float16, device=gpu)
+    xs[:, :K] = dev(x, gpu)
+    ws = torch.full((N, K // 2 + 16), 255, dtype=torch.uint8, device=gpu)
+    ws[:, :K // 2] = dev(wp, gpu)
+    big = torch.zeros((M, N + pad), dtype=torch.float16, device=gpu)
+    r = np.random.default_rng(2).standard_normal((M, N)).astype(np.float16)
+    out = big[:, :N]
+    out.copy_(dev(r, gpu))
+    with forced(mn, rows, parts):
+        mn.dequant_matmul(xs[:, :K], ws[:, :K // 2], dev(s, gpu), dev(z, gpu), g, "int4", epilogue="residual",
+                          residual=out, out=out)
+        assert mn.last_path() == "gemmn"
+    check(out.cpu().numpy(), acc, "residual", None, r, "strided")
+    assert (big[:, N:] == 0).all()
+
+
+# fp16 bit patterns: zero, subnormals, the ends of the normal scales that the
+# four-operation dequant covers (exponents 1..16), their neighbours, large ones
+SCALES = np.array([0x0000, 0x0001, 0x03FF, 0x0400, 0x0401, 0x1400, 0x2555, 0x3C00, 0x43FF, 0x4400, 0x5800, 0x6C00,
+                   0x8400, 0xA4D3, 0xC3FF, 0xC400], dtype=np.uint16)
+ZEROS = np.array([0x0000, 0x8000, 0x0001, 0x83FF, 0x2E66, 0xBC00, 0x5555, 0xE000], dtype=np.uint16)
+
+
+@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("qt", ["int4", "int8"])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_one_hot_selects_dequantized_weights(mn, gpu, rows, qt, mixed):
+    """Every dequantized weight equals the oracle's two-rounding one (up to
+    the sign of zero); `mixed`: scales outside the fast form's range among
+    the others, else none."""
+    rng = np.random.default_rng(5)
+    N, K, g, M = 320, 1024, 32, 256
+    pool = SCALES if mixed else SCALES[[3, 4, 5, 6, 7, 8, 12, 13, 14]]
+    s = pool[rng.integers(0, len(pool), (N, K // g))].view(np.float16)
+    if qt == "int8":   # keep the weights finite
+        s = np.clip(s.astype(np.float32), -255.0, 255.0).astype(np.float16)
+    if mixed:          # whole column blocks of both kinds, too
+        s[32:96] = np.float16(0.0123)
+    z = ZEROS[rng.integers(0, len(ZEROS), (N, K // g))].view(np.float16)
+    if qt == "int4":
+        wp = rng.integers(0, 256, (N, K // 2), dtype=np.uint8)
+        want = O.dequant_int4(wp, s, z, K, g)
+    else:
+        wp = rng.integers(-127, 128, (N, K), dtype=np.int16).astype(np.int8)
+        want = O.dequant_int8(wp, s, z, K, g)
+    assert np.isfinite(want).all()
+    order = rng.permutation(K)
+    with forced(mn, rows, 1):
+        for k0 in range(0, K, M):
+            ks = order[k0:k0 + M]
+            x = np.zeros((M, K), dtype=np.float16)
+            x[np.arange(M), ks] = 1.0
+            y = mn.dequant_matmul(dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, qt).cpu().numpy()
+            bad = y != want[:, ks].T
+            assert not bad.any(), f"{bad.sum()} differ, e.g. {y[bad][:4]} vs {want[:, ks].T[bad][:4]}"
+
+
+@pytest.mark.parametrize("M,K,N,g,qt,epi,want", [
+    (777, 4096, 3584, 128, "int4", "swiglu", "gemmn"),
+    (300, 8192, 2048, 32, "int4", None, "gemmn"),       # K parts; more groups than the other kernels' tables hold
+    (1100, 2048, 8192, 2048, "int8", "bias", "gemmn"),
+    (512, 3072, 5120, 128, "int4", None, "gemm16"),     # one round of the other kernel's tiles
+    (301, 4864, 896, 64, "int8", None, "gemmw_split"),
+])
+def test_routing(mn, gpu, M, K, N, g, qt, epi, want):
+    x, wp, s, z, g, acc = problem(M, K, N, g, qt, seed=K)
+    kw, b, r = epilogue_args(epi, M, N, gpu)
+    y = mn.dequant_matmul(dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, qt, **kw)
+    assert mn.last_path() == want, mn.last_path()
+    check(y.cpu().numpy(), acc, epi, b, r, want)
+
+
+def test_capture_and_shared_workspace(mn, gpu):
+    """K parts under capture: with the stream's workspace in place the graph
+    replays them; on a fresh stream a kernel without one runs.  The split-K
+    GEMV, whose counters share the workspace, stays right in between."""
+    M, K, N, g = 300, 8192, 2048, 128
+    x, wp, s, z, g, acc = problem(M, K, N, g, "int4", seed=4)
+    args = (dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, "int4")
+    v = O.make_int4_problem(1, 896, 4864, 64, seed=8)
+    vref = O.matmul_f32acc(v[0], O.dequant_int4(v[1], v[2], v[3], 896, 64))
+    vargs = tuple(dev(a, gpu) for a in v) + (64, "int4")
+    for warm in (True, False):
+        stream = torch.cuda.Stream(gpu)
+        stream.wait_stream(torch.cuda.current_stream(gpu))
+        if warm:
+            with torch.cuda.stream(stream):
+                mn.dequant_matmul(*args)
+                assert mn.last_path() == "gemmn"
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            y = mn.dequant_matmul(*args)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            check(y.cpu().numpy(), acc, what=f"replay warm={warm}")
+            with torch.cuda.stream(stream):
+                got = mn.dequant_matmul(*vargs)
+            torch.cuda.synchronize()
+            check(got.cpu().numpy(), vref, what="split-K GEMV between replays")
