@@ -12,6 +12,10 @@ are only reachable through QuantWeightCache in the reference,
 src/memory/quant_weight_cache.mm:65-153), ``quantize``, and the ``epilogue`` /
 ``bias`` keywords of ``dequant_matmul``.
 
+``dequant_matmul`` and ``matmul``'s vecmat route go through a native front
+(``_mq_torch``) when their tensors are plain and row-major and their arguments
+valid; everything else takes the checks and copies here.
+
 Every op launches a HIP kernel of libmetal_native_amd.so on the current torch
 stream and returns without synchronising, like the reference's lazy command
 buffers.  Outputs are fresh tensors owned by the caller.
@@ -25,7 +29,13 @@ import torch
 
 from . import _lib
 
+try:
+    from . import _mq_torch   # native front (csrc/mq_torch.cpp); after _lib, which loads the library it links
+except ImportError as e:
+    raise ImportError(f"{e}; run `python metal-native_amd/build.py` (or __graft_entry__.build()) first") from e
+
 _L = _lib.lib
+_raw_stream = torch._C._cuda_getCurrentRawStream
 
 
 class MetalNativeError(RuntimeError):
@@ -119,6 +129,13 @@ def dequant_matmul(activations: torch.Tensor, weights_packed: torch.Tensor, scal
     write instead of a new one.
     """
     op = "dequant_matmul"
+    if out is None and type(activations) is torch.Tensor and activations.is_cuda and epilogue in _EPILOGUES:
+        r = _mq_torch.dequant_matmul(activations, weights_packed, scales, zeros, group_size, quant_type == "int4",
+                                     _EPILOGUES[epilogue], bias, residual, _raw_stream(activations.get_device()))
+        if r is not None:
+            if type(r) is int:
+                _check(r)
+            return r
     _require_cuda(activations, "activations", op)
     if activations.dim() != 2:
         _invalid("dequant_matmul: activations must be 2D [M, K]")
@@ -339,6 +356,12 @@ def matmul(a: torch.Tensor, b: torch.Tensor, transpose_a: bool = False,
     they are computed by torch.matmul on the GPU (hipBLASLt).
     """
     op = "matmul"
+    if not transpose_a and type(a) is torch.Tensor and a.is_cuda:
+        r = _mq_torch.vecmat(a, b, bool(transpose_b), _raw_stream(a.get_device()))
+        if r is not None:
+            if type(r) is int:
+                _check(r)
+            return r
     if a.dim() < 2:
         _invalid("matmul: input 'a' must have at least 2 dimensions")
     if b.dim() < 2:
