@@ -149,12 +149,12 @@ bool gemm16_auto(const mq::LinearArgs& a) {
 
 // The many-row GEMM (mq_gemmn.hip), automatically: where its launch-time
 // model is at least 7 % below that of the kernel the shape would take
-// otherwise, and that one is 25 us or more (below, the models' errors exceed
-// the gain).  On 208 measured shapes (M = 32..4096) the choice is the faster
-// kernel or within 6 % of it on all but 5, e.g. M = 4096, K = 3584, N = 37888
-// int4 SwiGLU: 1.05 ms against 2.51; M = 777, K = 18944, N = 3584: 134 us
-// against 278; M = 512, K = 3072, N = 5120 stays with the 16x16x32 GEMM (23
-// against 35 us).
+// otherwise, and that one is 19 us or more (below, it was the slower one on
+// every shape).  On 208 shapes with M = 32..4096 and 148 with M = 17..512 the
+// choice is the faster kernel, or within 6 % of it, on all but 12: e.g. M =
+// 4096, K = 3584, N = 37888 int4 SwiGLU 1.05 ms against 2.51; M = 777, K =
+// 18944, N = 3584 134 us against 275; M = 37 there 28 against 33; M = 512,
+// K = 3072, N = 5120 stays with the 16x16x32 GEMM (23 against 35 us).
 mq::GemmnPlan gemmn_auto(const mq::LinearArgs& a, bool allow_split) {
   const int cus = num_cus_current();
   allow_split = allow_split && g_gemm_split.load() != 0;
@@ -167,7 +167,7 @@ mq::GemmnPlan gemmn_auto(const mq::LinearArgs& a, bool allow_split) {
   } else if (mq::gemmw_supported(a, cus)) {
     other = mq::gemmw_estimate(a, cus, allow_split);
   }
-  if (other < 25.0) return none;
+  if (other < 19.0) return none;
   const mq::GemmnPlan p = mq::gemmn_plan(a, cus, allow_split);
   return p.ok && p.us < 0.93 * other ? p : none;
 }
@@ -211,6 +211,7 @@ int choose_path(const mq::LinearArgs& a, bool noalloc) {
   // on 13 shapes, e.g. config 2 at M = 9 / 16: 19.0-19.7 / 21.6 us against
   // 25.0 / 25.4 us, K = 4096, N = 4096, M = 16: 8.3 against 12.0 us)
   if (a.M >= 5 && a.M <= 16 && mq::rstream_plan(a, num_cus_current()).ok) return PATH_RSTREAM;
+  if (gemmn_auto(a, !noalloc).ok) return PATH_GEMMN;
   // M = 9..16 with long rows the register-streamed plan declines: the prefill GEMM with K split over
   // workgroups beats the split-K GEMV (measured at K >= 8192 on 6 shapes at
   // M = 9, 12, 13-16: faster on all but K = 8192, N = 4096 (2-10 % slower
@@ -220,7 +221,6 @@ int choose_path(const mq::LinearArgs& a, bool noalloc) {
       mq::gemmw_supported(a, num_cus_current()) && mq::gemmw_ws_bytes(a, num_cus_current(), true) > 0)
     return PATH_TILED;
   if (decode_ok(a)) return PATH_DECODE;
-  if (gemmn_auto(a, !noalloc).ok) return PATH_GEMMN;
   if (prefill_ok(a)) return PATH_TILED;
   return PATH_GENERIC;
 }
@@ -716,13 +716,13 @@ MQ_API int mq_set_option(const char* key, int64_t value) {
     return MQ_SUCCESS;
   }
   if (std::strcmp(key, "gemm_rows") == 0) {
-    if (value != 0 && value != 128 && value != 256)
-      return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_rows must be 0, 128 or 256");
+    if (value != 0 && value != 64 && value != 128 && value != 256)
+      return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_rows must be 0, 64, 128 or 256");
     g_gemm_rows.store((int)value);
     return MQ_SUCCESS;
   }
   if (std::strcmp(key, "gemm_parts") == 0) {
-    if (value < 0 || value > 16) return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_parts must be 0..16");
+    if (value < 0 || value > 64) return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_parts must be 0..64");
     g_gemm_parts.store((int)value);
     return MQ_SUCCESS;
   }

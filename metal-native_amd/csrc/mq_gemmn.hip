@@ -1,6 +1,6 @@
 // Prefill dequant GEMM for many rows (int4 and int8 weights): C =
 // epi(A . deq(W)^T) on v_mfma_f32_32x32x16_f16, fp32 accumulation, one
-// rounding.  Tiles of 32*MB rows by 256 weight rows, MB = 8 or 4.
+// rounding.  Tiles of 32*MB rows by 256 weight rows, MB = 8, 4 or 2.
 //
 // Replaces dequant_matmul_int4_fp16 / dequant_matmul_int8_fp16
 // (shaders/matmul_dequant_kernel.metal:55-223, :351-479; dispatched at
@@ -112,8 +112,9 @@ gemmn_kernel(GNArgs p) {
   constexpr int NW = FMT == FMT_INT4 ? 2 : 4;   // weight loads per wave and K-tile
   constexpr int NL = NW / 2;                    // weight loads per block
   constexpr int NM = 2 * MB;                    // MFMAs per k-step
+  constexpr int DQ = (ND + 3) / 4;              // DMA instructions per k-step, at most
   // weight ring depth in K-tiles: 4, or 2 where registers are short
-  constexpr int WD = FMT == FMT_INT8 && MB == 4 ? 2 : 4;
+  constexpr int WD = FMT == FMT_INT8 && MB < 8 ? 2 : 4;
   // scale | zero << 16, [wave][iteration & 1][piece e][column ^ 8e]
   __shared__ uint32_t lds_sz[4][2][8 * 64];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -343,7 +344,7 @@ gemmn_kernel(GNArgs p) {
     auto first = [&](auto ic) {
       constexpr int I = decltype(ic)::value;
 #pragma unroll
-      for (int i = 0; i < (I < 3 ? ND : ND / 4); ++i) dma_one(I, slot(ic), i);   // (tile 3: the rest in the loop)
+      for (int i = 0; i < (I < 3 ? ND : DQ); ++i) dma_one(I, slot(ic), i);   // (tile 3: the rest in the loop)
       if (I < WD) load_w(I, wring[I % WD]);
     };
     first(std::integral_constant<int, 0>{});
@@ -365,7 +366,7 @@ gemmn_kernel(GNArgs p) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * ND + ND / 4 + (WD - 1) * NW) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * ND + DQ + (WD - 1) * NW) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
@@ -403,10 +404,9 @@ gemmn_kernel(GNArgs p) {
     // the slot that the barrier of tile t - 1 freed: a quarter of its refill
     // (K-tile t + 3) per k-step, so that the four waves' loads spread out
     auto refill = [&](int tt, u4* sl, int q, int m) {
-      constexpr int DQ = ND / 4;
 #pragma unroll
-      for (int i = 0; i < DQ; ++i)
-        if (2 + i * NM / DQ == m) dma_one(tt, sl, DQ * q + i);
+      for (int i = 0; i < ND; ++i)
+        if (i * 4 / ND == q && 2 + (i % DQ) * NM / DQ == m) dma_one(tt, sl, i);
     };
     u4* const prv = slot(std::integral_constant<int, (R + 3) & 3>{});
     constexpr auto late = std::false_type{};
@@ -642,8 +642,10 @@ constexpr size_t kCntBytesN = 65536;
 //    us when all CUs run (the clock drops under the load).
 //  * 128 rows: two workgroups fit a CU; a K-tile takes 0.77-1.05 us alone,
 //    2.02 us in each of two.
+//  * 64 rows: two workgroups fit a CU; a K-tile takes 0.71 us alone, 1.05 us in
+//    each of two (1414 launches, M = 17..512, 7 % rms).
 //  * K parts: their sums are written and read once, 0.145 us per MB.
-double estimate(int mb, int64_t wgs, int ktp, double part_mb, int cus) {
+double estimate(int mb, int64_t wgs, int ktp, double part_mb, double weight_mb, int cus) {
   const double split = part_mb > 0.0 ? 1.0 : 0.0;
   if (mb == 8) {
     const double rounds = (double)wgs / cus;
@@ -653,6 +655,11 @@ double estimate(int mb, int64_t wgs, int ktp, double part_mb, int cus) {
   }
   const int64_t slots = 2 * (int64_t)cus;
   const int64_t full = wgs / slots, rem = wgs - full * slots;
+  if (mb == 2) {
+    double t = (full + (rem > cus ? 1 : 0)) * (ktp * 1.053 - 1.57);
+    if (rem > 0 && rem <= cus) t += ktp * 0.709 * (1.0 + 0.009 * (double)rem / cus) - 1.57;
+    return 6.72 + std::max(0.0, t) + 0.09 * weight_mb + split * 2.46 + 0.231 * part_mb;
+  }
   double t = 8.05 + full * (1.55 + ktp * 2.02);
   if (rem > cus) t += 1.55 + ktp * (0.77 + 1.25 * (0.6 + 0.4 * (double)(rem - cus) / cus));
   else if (rem > 0) t += 1.55 + ktp * 0.77 * (1.0 + 0.36 * (double)rem / cus);
@@ -668,18 +675,19 @@ GemmnPlan gemmn_plan(const LinearArgs& a, int cus, bool allow_split, int mb, int
   const int F = swi ? a.F : a.N;
   const int KT = (a.K + 63) / 64;
   const int64_t ld = (int64_t)((F + 7) & ~7) * (swi ? 2 : 1);
-  for (int m = 4; m <= 8; m += 4) {
-    if (mb && m != mb) continue;
+  const double wmb = (double)a.N * a.K * (a.fmt == FMT_INT4 ? 0.5e-6 : 1e-6);
+  for (int m = 2; m <= 8; m *= 2) {
+    if (mb ? m != mb : m == 2 && a.M > 320) continue;   // (64 rows: not the fastest beyond, and not modelled)
     const int64_t tiles = (int64_t)((a.M + 32 * m - 1) / (32 * m)) * ((F + (swi ? 127 : 255)) / (swi ? 128 : 256));
-    for (int q = 1; q <= 16; ++q) {
+    for (int q = 1; q <= (m == 2 ? 64 : 16); ++q) {
       if (kp && q != kp) continue;
       const int ktp = (KT + q - 1) / q, KP = (KT + ktp - 1) / ktp;
-      if (!kp && KP > 1 && (KP != q || ktp < 4 || tiles * KP > 4 * (int64_t)cus)) continue;
+      if (!kp && KP > 1 && (KP != q || ktp < (m == 2 ? 3 : 4) || tiles * KP > 4 * (int64_t)cus)) continue;
       if (KP > 1 && !allow_split) continue;
       if (tiles * KP > 0x7fffffff / 256) continue;
       const size_t part = KP > 1 ? (size_t)KP * a.M * ld * 4 : 0;
       if (part > kMaxPartBytes) continue;
-      const double t = estimate(m, tiles * KP, ktp, 2.0 * (double)part / 1e6, cus);
+      const double t = estimate(m, tiles * KP, ktp, 2.0 * (double)part / 1e6, wmb, cus);
       if (!best.ok || t < best.us) best = GemmnPlan{m, KP, ktp, part ? kCntBytesN + part : 0, t, true};
     }
   }
@@ -719,8 +727,11 @@ hipError_t gemmn_launch(const LinearArgs& a, const GemmnPlan& pl, void* ws, hipS
   k.w_bytes = (uint32_t)((int64_t)(a.N - 1) * a.ldw + wrow);
   k.s_bytes = (uint32_t)((int64_t)a.N * a.G * 2);
   k.z_bytes = a.zeros ? k.s_bytes : 0u;
-  if (a.fmt == FMT_INT4) return mb == 8 ? launch_mb<FMT_INT4, 8>(k, swi, nwg, s) : launch_mb<FMT_INT4, 4>(k, swi, nwg, s);
-  return mb == 8 ? launch_mb<FMT_INT8, 8>(k, swi, nwg, s) : launch_mb<FMT_INT8, 4>(k, swi, nwg, s);
+  if (a.fmt == FMT_INT4)
+    return mb == 8 ? launch_mb<FMT_INT4, 8>(k, swi, nwg, s)
+         : mb == 4 ? launch_mb<FMT_INT4, 4>(k, swi, nwg, s) : launch_mb<FMT_INT4, 2>(k, swi, nwg, s);
+  return mb == 8 ? launch_mb<FMT_INT8, 8>(k, swi, nwg, s)
+       : mb == 4 ? launch_mb<FMT_INT8, 4>(k, swi, nwg, s) : launch_mb<FMT_INT8, 2>(k, swi, nwg, s);
 }
 
 }  // namespace mq

@@ -560,7 +560,7 @@ bool sz_table_fits(const LinearArgs& a, int BN) {
 // measured launches (int4, M = 17..128, K = 2048..18944): per-wave K-tiles
 // times the tile's MFMA, dequant and activation work, rounds of workgroups
 // over the CUs, and for K parts a fixed cost plus the last arriver's reads of
-// the parts.  (14 % rms over a further 80 launches up to M = 4096.)
+// the parts.
 double launch_us(int K, int MB, int NB, int64_t tiles, int KP, int cus) {
   const double per = std::ceil(K / 64.0) / KP / 4.0;
   const double rounds = std::ceil((double)(tiles * KP) / cus);
@@ -706,9 +706,22 @@ bool gemmw_supported(const LinearArgs& a, int cus) {
 
 size_t gemmw_ws_bytes(const LinearArgs& a, int cus, bool allow_split) { return plan(a, cus, allow_split).ws_bytes; }
 
+// Per format, fitted to 117 (int4) and 62 (int8) measured launches up to M =
+// 4096 (10 % and 7 % rms; launch_us, which only ranks this kernel's own
+// tilings, is 14 % and 10 % off there): a round of workgroups costs a fixed
+// time and its per-wave K-tiles times the work of an MB x NB tile.
 double gemmw_estimate(const LinearArgs& a, int cus, bool allow_split) {
   const WPlan p = plan(a, cus, allow_split);
-  return p.ok ? launch_us(a.K, p.MB, p.NB, (int64_t)p.nbm * p.nbn, p.KP, cus) : 0.0;
+  if (!p.ok) return 0.0;
+  const bool i4 = a.fmt == FMT_INT4;
+  const double c0 = i4 ? -2.05 : 1.03, c1 = i4 ? 7.63 : 6.93, k0 = i4 ? 19.25 : 18.65, kmn = i4 ? 4.94 : 4.78;
+  const double kn = i4 ? -9.43 : -9.11, km = i4 ? -9.66 : -9.42, load = i4 ? 0.006 : 0.054;
+  const double s0 = i4 ? 1.43 : -1.70, s1 = i4 ? 0.207 : 0.258;
+  const double per = std::ceil(a.K / 64.0) / p.KP / 4.0, mn = (double)p.MB * p.NB;
+  const double r = (double)((int64_t)p.nbm * p.nbn * p.KP) / cus;
+  const double rounds = std::ceil(r) <= 3.0 ? std::ceil(r) : r + 0.5;
+  const double tile = k0 + kmn * mn + kn * p.NB + km * p.MB + load * mn * std::min(1.0, std::max(0.0, r - 0.5));
+  return c0 + rounds * (c1 + per * tile) + (p.KP > 1 ? s0 + s1 * p.KP * mn : 0.0);
 }
 
 hipError_t gemmw_launch(const LinearArgs& a, int cus, void* ws, hipStream_t s, bool allow_split) {

@@ -125,7 +125,7 @@ double gemm16_estimate(const LinearArgs& a, int num_cus);   // launch time (us)
 hipError_t gemm16_launch(const LinearArgs& a, hipStream_t s, uint64_t* trace);
 
 // GEMM for many rows (32x32x16 MFMA, waves side by side along N, shared
-// activation tiles, no workspace): 32 * mb rows per tile, mb = 4 or 8.
+// activation tiles, no workspace): 32 * mb rows per tile, mb = 2, 4 or 8.
 bool gemmn_supported(const LinearArgs& a);
 // K may be split over KP workgroups per tile, whose fp32 sums (ws_bytes, need
 // not be cleared) a second kernel adds up.

@@ -95,7 +95,7 @@ def epilogue_args(epi, M, N, gpu):
     return ({"epilogue": epi} if epi else {}), None, None
 
 
-@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("rows", [64, 128, 256])
 @pytest.mark.parametrize("parts", [1, 3])
 @pytest.mark.parametrize("M,K,N,g,qt,epi", [
     (1, 64, 2, 32, "int4", None),              # one K-tile, one row
@@ -120,7 +120,7 @@ def test_against_oracle(mn, gpu, rows, parts, M, K, N, g, qt, epi):
         assert torch.equal(run(), y)   # a fixed summation order
 
 
-@pytest.mark.parametrize("rows,parts", [(128, 1), (256, 1), (128, 2)])
+@pytest.mark.parametrize("rows,parts", [(64, 1), (128, 1), (256, 1), (64, 2), (128, 2)])
 @pytest.mark.parametrize("pad", [8, 3])
 def test_strided_operands(mn, gpu, rows, parts, pad):
     """Activations, weights and output as column ranges of wider tensors, the
@@ -150,7 +150,7 @@ SCALES = np.array([0x0000, 0x0001, 0x03FF, 0x0400, 0x0401, 0x1400, 0x2555, 0x3C0
 ZEROS = np.array([0x0000, 0x8000, 0x0001, 0x83FF, 0x2E66, 0xBC00, 0x5555, 0xE000], dtype=np.uint16)
 
 
-@pytest.mark.parametrize("rows", [128, 256])
+@pytest.mark.parametrize("rows", [64, 128, 256])
 @pytest.mark.parametrize("qt", ["int4", "int8"])
 @pytest.mark.parametrize("mixed", [False, True])
 def test_one_hot_selects_dequantized_weights(mn, gpu, rows, qt, mixed):
@@ -188,8 +188,9 @@ def test_one_hot_selects_dequantized_weights(mn, gpu, rows, qt, mixed):
     (777, 4096, 3584, 128, "int4", "swiglu", "gemmn"),
     (300, 8192, 2048, 32, "int4", None, "gemmn"),       # K parts; more groups than the other kernels' tables hold
     (1100, 2048, 8192, 2048, "int8", "bias", "gemmn"),
+    (37, 18944, 3584, 128, "int4", "residual", "gemmn"),
     (512, 3072, 5120, 128, "int4", None, "gemm16"),     # one round of the other kernel's tiles
-    (301, 4864, 896, 64, "int8", None, "gemmw_split"),
+    (64, 3104, 256, 32, "int4", None, "gemmw_split"),
 ])
 def test_routing(mn, gpu, M, K, N, g, qt, epi, want):
     x, wp, s, z, g, acc = problem(M, K, N, g, qt, seed=K)
