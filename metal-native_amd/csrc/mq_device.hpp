@@ -147,6 +147,52 @@ __device__ __forceinline__ h8 dq_int4_dword_perm_r(uint32_t d, h2 s, h2 z, uint3
   return r;
 }
 
+// The same eight weights in 13 VALU ops instead of 17, without forming q - 8.
+// A nibble alone in an fp16 (the other bits zero) is the subnormal q * 2^-24,
+// or q * 2^-20 four bits up.  With s = (1 + m) 2^(e - 15) and S = (1 + m) 2^10,
+//   fma(q * 2^-20, S, -8 (1 + m) 2^-10) = RNE((q - 8) (1 + m) 2^-10):
+// the addend is exact and the result normal, so its one rounding is that of
+// RNE((q - 8) s), P = 2^(e - 5) times smaller.  Then fma(., P, -z) =
+// RNE(RNE((q - 8) s) - z), the reference's two roundings.  The low nibbles
+// take 2^-14 in place of 2^-10 and 16 P in place of P.  Valid for exponents
+// 1 <= e <= 16, i.e. 2^-14 <= |s| < 4; other scales take the direct form.
+struct FastDq {
+  h2 S;   // low half: S
+  h2 C;   // addends of the low nibbles (low half) and the high nibbles
+  h2 P;   // 16 P | P
+  h2 e;   // s | z
+};
+__device__ __forceinline__ FastDq fast_dq(uint32_t sz) {
+  FastDq f;
+  f.e = as_h2(sz);
+  f.S = as_h2((sz & 0xFFFF83FFu) | (25u << 10));
+  f.C = __builtin_shufflevector(f.S, f.S, 0, 0) * as_h2(0x80808008u);   // times -2^-21 | -2^-17
+  f.P = as_h2(__umul24(sz & 0x7C00u, 0x10001u) + 0x28003800u);
+  return f;
+}
+__device__ __forceinline__ h8 dq_int4_dword_perm_fast(uint32_t d, const FastDq& f, uint32_t mlo, uint32_t mhi) {
+  const h2 S = __builtin_shufflevector(f.S, f.S, 0, 0), z = __builtin_shufflevector(f.e, f.e, 1, 1);
+  const h2 Cl = __builtin_shufflevector(f.C, f.C, 0, 0), Ch = __builtin_shufflevector(f.C, f.C, 1, 1);
+  const h2 Pl = __builtin_shufflevector(f.P, f.P, 0, 0), Ph = __builtin_shufflevector(f.P, f.P, 1, 1);
+  const uint32_t d8 = d >> 8;
+  auto lo = [&](uint32_t v) { return __builtin_elementwise_fma(__builtin_elementwise_fma(as_h2(v & mlo), S, Cl), Pl, -z); };
+  auto hi = [&](uint32_t v) { return __builtin_elementwise_fma(__builtin_elementwise_fma(as_h2(v & mhi), S, Ch), Ph, -z); };
+  h8 r;
+  r.s01 = lo(d);    // k0, k4
+  r.s23 = hi(d);    // k1, k5
+  r.s45 = lo(d8);   // k2, k6
+  r.s67 = hi(d8);   // k3, k7
+  return r;
+}
+// Range test of scale pairs: m starts at 0, fast_scale_max folds in two
+// scales, fast_scale_bad(m) tells whether any had an exponent outside 1..16.
+typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t fast_scale_max(uint32_t m, uint32_t s2) {
+  const us2 x = __builtin_bit_cast(us2, s2 & 0x7C007C00u) - (us2){0x0400, 0x0400};
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2, m), x));
+}
+__device__ __forceinline__ bool fast_scale_bad(uint32_t m) { return (m & 0xC000C000u) != 0; }
+
 // Eight int4 weights in natural k order (used where the output is stored,
 // i.e. the dequantize op).  v_perm_b32 copies byte b into bytes 0 and 2 so
 // the two nibbles of one byte land in the two fp16 halves.

@@ -43,7 +43,9 @@
 #include "mq_launch.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
+#include <type_traits>
 
 namespace mq {
 namespace {
@@ -99,6 +101,12 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   constexpr int BPK2 = (FMT == FMT_INT4) ? 1 : (FMT == FMT_INT8 ? 2 : 4);  // 2 x bytes per k
   extern __shared__ __align__(16) unsigned char smem[];
 
+  // The 13-op dequant, in the twelve-wave builds: with its range test and a
+  // second loop for other scales the start of a launch is ~0.3 us longer, and
+  // the stream of 34 MB and more shorter by more than that (7B gate/up 17.9 ->
+  // 17.4 us, lm_head 57.2 -> 54.2, down 11.8 -> 11.5; QKV and o_proj, eight
+  // waves, 7.7 -> 8.0 and 5.74 -> 5.80 us).
+  constexpr bool FASTDQ = FMT == FMT_INT4 && NW == kNWBig;
   constexpr int NT = 64 * NW;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -111,7 +119,10 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   uint32_t* szl = (uint32_t*)(smem + p.off_sz);       // [regions][8 snp]: s | z << 16
   float* scr = (float*)(smem + p.off_scr) + w * 256;  // per wave [16][16]
   float* slots = (float*)(smem + p.off_slot);         // [NW][maxT][M*RPW]
-  int* wft = (int*)(smem + p.off_wft);                // [NW] first tile of each wave's unit range
+  // [NW] first tile of each wave's unit range; FASTDQ: bit 31 set when a scale
+  // that the wave staged needs the direct dequant
+  int* wft = (int*)(smem + p.off_wft);
+  uint32_t smax = 0;   // FASTDQ: range test of the staged scales
 
   const int nl = lane & 15, gi = lane >> 4;
   const int r = nl % RPW, sh = nl / RPW;              // weight row in tile, K shift
@@ -269,6 +280,19 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
       const int idx = base + tid + e * NT;
       if (e < cnt && idx < nps) {
         const u4 a = sv[e], z = zv[e];
+        if (FASTDQ) {
+          const uint32_t off = (uint32_t)(idx < snp ? pb0 + idx : pb1 - snp + idx) * 16u;
+          if (off + 16u <= sz_real) {
+            smax = fast_scale_max(fast_scale_max(fast_scale_max(fast_scale_max(smax, a.x), a.y), a.z), a.w);
+          } else {   // the last entries of the arrays: those past the end count as 1.0
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+              const uint32_t o = off + 4u * h;
+              smax = fast_scale_max(smax, o + 4u <= sz_real ? a[h] : o + 2u <= sz_real ? (a[h] & 0xFFFFu) | 0x3C000000u
+                                                                                       : 0x3C003C00u);
+            }
+          }
+        }
         *(u4*)(szl + 8 * idx) = (u4){__builtin_amdgcn_perm(z.x, a.x, 0x05040100u), __builtin_amdgcn_perm(z.x, a.x, 0x07060302u),
                                      __builtin_amdgcn_perm(z.y, a.y, 0x05040100u), __builtin_amdgcn_perm(z.y, a.y, 0x07060302u)};
         *(u4*)(szl + 8 * idx + 4) = (u4){__builtin_amdgcn_perm(z.z, a.z, 0x05040100u), __builtin_amdgcn_perm(z.z, a.z, 0x07060302u),
@@ -366,6 +390,10 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   }
 #pragma unroll
   for (int d = kPre; d < kD; ++d) raw[d] = wload();
+  {
+    const int bad = FASTDQ && __builtin_amdgcn_ballot_w64(fast_scale_bad(smax)) != 0 ? INT_MIN : 0;
+    if (lane == 0) wft[w] = (u0 / KS) | bad;   // the tiles are read by the slot sums after the final barrier
+  }
   // LDS barrier that leaves the weight loads in flight
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
@@ -374,13 +402,13 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   // half's fragments RPW rows further down, the same dequantized weights)
   const int xrow = min(r, M - 1) * p.XS;
   const int xdh = (min(r + RPW, M - 1) - min(r, M - 1)) * p.XS;
-  uint32_t mlo = 0x000F000Fu, mhi = 0x00F000F0u;
-  asm volatile("" : "+v"(mlo), "+v"(mhi));  // keep the nibble masks in VGPRs
+  uint32_t mlo = 0x000F000Fu, mhi = 0x00F000F0u, slo = mlo, shi = mhi;
+  asm volatile("" : "+v"(mlo), "+v"(mhi));  // the direct form's v_and_or_b32 wants its nibble masks in VGPRs
+  asm volatile("" : "+s"(slo), "+s"(shi));  // the fast form's v_and_b32 in SGPRs
   const uint32_t magic = 0x64006400u;
 
   int ct = u0 / KS, cj = u0 - ct * KS;   // consume cursor (tile, step)
   const int ft = ct;                      // first tile of this wave
-  if (lane == 0) wft[w] = ft;   // read by the slot sums after the final barrier
   // scale entry of the lane's row and group: the step advances it by a
   // uniform KSTEP / g groups.  In a row's last step, lanes whose k lies past
   // K would reach the next row's entries: they keep their own row's last
@@ -431,9 +459,12 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
     }
   };
 
-  auto step = [&](const u4 v) {
+  auto step = [&](auto fastc, const u4 v) {
+    constexpr bool FAST = decltype(fastc)::value;
+    FastDq fd;
+    if constexpr (FAST) fd = fast_dq(szl[sa]);
     h2 s2 = (h2){(_Float16)0.f, (_Float16)0.f}, z2 = s2;
-    if (FMT != FMT_F16) {
+    if (FMT != FMT_F16 && !FAST) {
       // broadcast halves: the packed ops' operand selectors read them in place
       const h2 e = as_h2(szl[sa]);
       s2 = __builtin_shufflevector(e, e, 0, 0);
@@ -444,7 +475,8 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
       h8 bq;
       if (FMT == FMT_INT4) {
         const uint32_t dw = (j == 0) ? v.x : (j == 1) ? v.y : (j == 2) ? v.z : v.w;
-        bq = dq_int4_dword_perm_r(dw, s2, z2, mlo, mhi, magic);
+        if constexpr (FAST) bq = dq_int4_dword_perm_fast(dw, fd, slo, shi);
+        else bq = dq_int4_dword_perm_r(dw, s2, z2, mlo, mhi, magic);
       } else if (FMT == FMT_INT8) {
         const uint32_t d0 = (j == 0) ? v.x : v.z;
         const uint32_t d1 = (j == 0) ? v.y : v.w;
@@ -468,31 +500,42 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   // units are not left to one wave that cannot hide the load latency alone
   __builtin_amdgcn_s_setprio(3);
   const int q1 = nu >> 2, q2 = nu >> 1, q3 = (3 * nu) >> 2;
-  for (int base = 0; base < nu; base += kD) {
+  auto stream = [&](auto fastc) __attribute__((always_inline)) {
+    for (int base = 0; base < nu; base += kD) {
 #pragma unroll
-    for (int d = 0; d < kD; ++d) {
-      if (base + d < nu) {
-        if (base + d == q1) __builtin_amdgcn_s_setprio(2);
-        if (base + d == q2) __builtin_amdgcn_s_setprio(1);
-        if (base + d == q3) __builtin_amdgcn_s_setprio(0);
-        step(raw[d]);
-        if constexpr (XCONST) xa += XADV;
-        sa += sadv;
-        const bool last = base + d == nu - 1;
-        if (++cj == KS || last) {
-          flush();
-          if (cj == KS) {
-            cj = 0;
-            ++ct;
-            xa = xs + xrow + xswz(klane);
-            sa = sz_ent(ct) + sl + ks0 * sadv;
+      for (int d = 0; d < kD; ++d) {
+        if (base + d < nu) {
+          if (base + d == q1) __builtin_amdgcn_s_setprio(2);
+          if (base + d == q2) __builtin_amdgcn_s_setprio(1);
+          if (base + d == q3) __builtin_amdgcn_s_setprio(0);
+          step(fastc, raw[d]);
+          if constexpr (XCONST) xa += XADV;
+          sa += sadv;
+          const bool last = base + d == nu - 1;
+          if (++cj == KS || last) {
+            flush();
+            if (cj == KS) {
+              cj = 0;
+              ++ct;
+              xa = xs + xrow + xswz(klane);
+              sa = sz_ent(ct) + sl + ks0 * sadv;
+            }
           }
+          if constexpr (!XCONST) xa = xs + xrow + xswz(cj * KSTEP + klane);
+          clamp_last();
         }
-        if constexpr (!XCONST) xa = xs + xrow + xswz(cj * KSTEP + klane);
-        clamp_last();
+        raw[d] = wload();
       }
-      raw[d] = wload();
     }
+  };
+  if constexpr (FASTDQ) {
+    int any = 0;
+#pragma unroll
+    for (int ww = 0; ww < NW; ++ww) any |= wft[ww];
+    if (__builtin_amdgcn_readfirstlane(any) >= 0) stream(std::true_type{});
+    else stream(std::false_type{});
+  } else {
+    stream(std::false_type{});
   }
   __syncthreads();
 
@@ -510,6 +553,9 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
     for (int ww = 0; ww < NW; ww += 4) {
       const int4 f4 = *(const int4*)(wft + ww);
       fw[ww] = f4.x; fw[ww + 1] = f4.y; fw[ww + 2] = f4.z; fw[ww + 3] = f4.w;
+      if (FASTDQ)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) fw[ww + e] &= INT_MAX;
     }
     float sv[NW];
     bool use[NW];
