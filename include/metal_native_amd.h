@@ -210,6 +210,28 @@ MQ_API int mq_attention_decode_rope_f16(const void* qkv, const float* cos_table,
                                         int32_t kv_heads, int32_t head_dim, int64_t max_len, float scale,
                                         void* stream);
 
+/* The same attention over four workgroups per head, and the o_proj that
+ * combines their partials while it stages them (no reference counterpart):
+ * parts is a buffer of mq_attention_parts_size(heads, head_dim) bytes, 16-byte
+ * aligned (fp32 [heads][4][head_dim] partial outputs, then [heads][4] pairs of
+ * running maximum and weight sum).  mq_attention_parts_dequant_matmul: C[N] =
+ * half(attention output) . deq(W)^T, W int4 [N, heads * head_dim].  Both run
+ * where mq_attention_parts_supported (one int4 row of at most 8192 columns;
+ * caches of more than 256 positions at head_dim 128, 512 at 64: the split
+ * gains nothing in shorter ones); otherwise they return 4 and the caller runs
+ * mq_attention_decode_rope_f16 and mq_dequant_matmul. */
+MQ_API int64_t mq_attention_parts_size(int32_t heads, int32_t head_dim);
+MQ_API int mq_attention_parts_supported(int64_t N, int32_t heads, int32_t head_dim, int64_t max_len, int32_t group_size,
+                                        int32_t quant_type);
+MQ_API int mq_attention_decode_rope_parts_f16(const void* qkv, const float* cos_table, const float* sin_table,
+                                              const int64_t* pos, void* k_cache, void* v_cache, void* parts,
+                                              int32_t heads, int32_t kv_heads, int32_t head_dim, int64_t max_len,
+                                              float scale, void* stream);
+MQ_API int mq_attention_parts_dequant_matmul(const void* parts, int32_t heads, int32_t head_dim,
+                                             const void* weights_packed, int64_t ldw_bytes, const void* scales,
+                                             const void* zeros, void* C, int64_t N, int32_t group_size,
+                                             int32_t quant_type, void* stream);
+
 /* Greedy decode tail in one launch (decoder glue, no reference counterpart;
  * replaces torch.argmax + the embedding lookup + the position update of a
  * decode loop): token[0] = argmax(logits[vocab]) in torch.argmax order (NaN

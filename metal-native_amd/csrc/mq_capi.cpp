@@ -665,6 +665,68 @@ MQ_API int mq_attention_decode_rope_f16(const void* qkv, const float* cos_table,
   return MQ_SUCCESS;
 }
 
+MQ_API int64_t mq_attention_parts_size(int32_t heads, int32_t head_dim) {
+  if (heads < 1 || (head_dim != 64 && head_dim != 128)) return -1;
+  return (int64_t)mq::attn_parts_floats(heads, head_dim) * 4;
+}
+
+MQ_API int mq_attention_decode_rope_parts_f16(const void* qkv, const float* cos_table, const float* sin_table,
+                                              const int64_t* pos, void* k_cache, void* v_cache, void* parts,
+                                              int32_t heads, int32_t kv_heads, int32_t head_dim, int64_t max_len,
+                                              float scale, void* stream) {
+  if (!qkv || !cos_table || !sin_table || !pos || !k_cache || !v_cache || !parts)
+    return fail(MQ_INVALID_ARGUMENT, "attention_decode_rope_parts: null pointer argument");
+  if (heads < 1 || kv_heads < 1 || heads % kv_heads || max_len < 1 ||
+      !mq::attn_parts_supported(heads, head_dim, max_len) || ((uintptr_t)parts & 15))
+    return fail(MQ_INVALID_ARGUMENT,
+                "attention_decode_rope_parts: bad shape (head_dim 64 or 128, max_len > 32768 / head_dim)");
+  hipError_t e = mq::attn_parts_launch(qkv, cos_table, sin_table, pos, k_cache, v_cache, (float*)parts, heads, kv_heads,
+                                       head_dim, max_len, scale, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "attention_decode_rope_parts: kernel launch failed");
+  return MQ_SUCCESS;
+}
+
+MQ_API int mq_attention_parts_dequant_matmul(const void* parts, int32_t heads, int32_t head_dim,
+                                             const void* weights_packed, int64_t ldw_bytes, const void* scales,
+                                             const void* zeros, void* C, int64_t N, int32_t group_size,
+                                             int32_t quant_type, void* stream) {
+  if (heads < 1 || head_dim < 1) return fail(MQ_INVALID_ARGUMENT, "attention_parts_dequant_matmul: bad shape");
+  const int64_t K = (int64_t)heads * head_dim;
+  mq::LinearArgs a{};
+  int rc = build_args(a, 1, N, K, group_size, quant_type, MQ_EPILOGUE_NONE);
+  if (rc != MQ_SUCCESS) return rc;
+  alignas(16) static const uint64_t kAligned[2] = {0, 0};   // stands in for A, which this form does not read
+  a.A = kAligned; a.lda = K;
+  a.W = weights_packed; a.ldw = ldw_bytes;
+  a.scales = scales; a.zeros = zeros;
+  a.C = C; a.ldc = N;
+  a.prenorm = 2; a.pre_parts = parts; a.pre_dim = head_dim;
+  if (!parts || !weights_packed || !scales || !C)
+    return fail(MQ_INVALID_ARGUMENT, "attention_parts_dequant_matmul: null pointer argument");
+  if (ldw_bytes < (quant_type == MQ_QUANT_INT4 ? K / 2 : K))
+    return fail(MQ_INVALID_ARGUMENT, "attention_parts_dequant_matmul: weight rows too short");
+  const mq::RowsPlan pl = mq::rows_plan(a, num_cus_current());
+  if (!pl.ok) return fail(MQ_INVALID_ARGUMENT, "attention_parts_dequant_matmul: shape not supported by the fused kernel");
+  hipError_t e = mq::rows_launch(a, pl, nullptr, (hipStream_t)stream);
+  if (e != hipSuccess) return hip_fail(e, "attention_parts_dequant_matmul: kernel launch failed");
+  g_last_path = PATH_ROWS;
+  return MQ_SUCCESS;
+}
+
+MQ_API int mq_attention_parts_supported(int64_t N, int32_t heads, int32_t head_dim, int64_t max_len, int32_t group_size,
+                                        int32_t quant_type) {
+  if (heads < 1 || max_len < 1 || N < 1 || !mq::attn_parts_supported(heads, head_dim, max_len)) return 0;
+  mq::LinearArgs a{};
+  const int64_t K = (int64_t)heads * head_dim;
+  if (build_args(a, 1, N, K, group_size, quant_type, MQ_EPILOGUE_NONE) != MQ_SUCCESS) return 0;
+  alignas(16) static const uint64_t kAligned[2] = {0, 0};
+  a.A = a.W = a.scales = kAligned;
+  a.lda = K;
+  a.ldw = quant_type == MQ_QUANT_INT4 ? K / 2 : K;
+  a.prenorm = 2; a.pre_parts = kAligned; a.pre_dim = head_dim;
+  return mq::rows_plan(a, num_cus_current()).ok ? 1 : 0;
+}
+
 MQ_API int64_t mq_argmax_embed_workspace_size(int64_t vocab) {
   if (vocab < 1 || vocab > (int64_t)INT32_MAX - 2048) return -1;
   return (int64_t)mq::argmax_embed_workspace(vocab);

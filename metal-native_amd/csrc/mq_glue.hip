@@ -294,10 +294,13 @@ __global__ __launch_bounds__(128) void attn_combine_kernel(const float* ws, _Flo
 // new token's k and v are taken from registers (its cache row is stale until
 // written) and written into the caches by the workgroup of the first query
 // head of each KV group (no other workgroup reads position pos).
-template <int D>
+// PARTS: kAttnParts workgroups per head, each leaving its partial output and
+// (max, exp-sum) for the kernel that reads them (the o_proj's staging).
+template <int D, bool PARTS>
 __global__ __launch_bounds__(768) void attn_head_d_kernel(const _Float16* qkv, const float* cos_t, const float* sin_t,
                                                           const int64_t* pos_p, _Float16* kc, _Float16* vc,
-                                                          _Float16* out, int H, int KVH, int64_t L, float scale) {
+                                                          _Float16* out, float* parts, int H, int KVH, int64_t L,
+                                                          float scale) {
   // floating-point attention (checked against a tolerance, not bit-exact):
   // multiply-adds may fuse here, unlike in the dequant arithmetic
 #pragma clang fp contract(fast)
@@ -325,12 +328,22 @@ __global__ __launch_bounds__(768) void attn_head_d_kernel(const _Float16* qkv, c
       vv[i] = *(const h8*)(vc + off);
     }
   };
-  load_rows(w);   // NW <= nsplit: every wave has a first split
+  // PARTS: workgroup (h, sp) takes every kAttnParts-th step, so that a short
+  // context spreads over the workgroups too.  The first 16 steps are fetched
+  // before the position is known (a wave's loads past the cache are clamped
+  // and not used); the others only where the context reaches them: with every
+  // step fetched, position 30 of a 4096-position cache took 1.6 us longer.
+  constexpr int S = PARTS ? kAttnParts : 1;
+  const int sp = PARTS ? blockIdx.y : 0;
+  const int c0 = w * S + sp;
+  const bool early = !PARTS || c0 < 16;
+  if (early) load_rows(c0);
   // positions outside [0, L): no cache write, attention over the cache rows
   // that exist, the nearest table row (no access outside any buffer)
   const int64_t pos = *pos_p;
   const bool in = pos >= 0 && pos < L;
   const int n = positions_in_cache(pos, L);
+  if (!early && c0 * SUB < n) load_rows(c0);
   const int64_t pt = pos < 0 ? 0 : (pos < L ? pos : L - 1);
   const float* cs = cos_t + pt * D;
   const float* sn = sin_t + pt * D;
@@ -350,7 +363,7 @@ __global__ __launch_bounds__(768) void attn_head_d_kernel(const _Float16* qkv, c
       const _Float16 kn = rope(krow, j), vn = vsrc[j];
       kn16[j] = kn;
       vn16[j] = vn;
-      if (in && h % grp == 0) {
+      if (in && h % grp == 0 && sp == 0) {
         kc[prow + j] = kn;
         vc[prow + j] = vn;
       }
@@ -361,7 +374,7 @@ __global__ __launch_bounds__(768) void attn_head_d_kernel(const _Float16* qkv, c
 #pragma unroll
   for (int e = 0; e < 4; ++e) qh[e] = (h2){(_Float16)qs[8 * q + 2 * e], (_Float16)qs[8 * q + 2 * e + 1]};
   float m_run = -INFINITY, l_run = 0.f, o_run[8] = {};
-  for (int c = w; c < nsplit; c += NW) {
+  for (int c = c0; c < nsplit; c += NW * S) {
     const int t0 = c * SUB;
     if (t0 >= n) break;   // this and the wave's later steps lie past the new token
     if (in && pos >= t0 && pos < t0 + SUB) {   // the split holding the new token: its row from registers
@@ -413,7 +426,7 @@ __global__ __launch_bounds__(768) void attn_head_d_kernel(const _Float16* qkv, c
     // the next split's rows: issued once this split's are consumed (the fence
     // keeps the loads from being hoisted above the uses, doubling the rows live)
     asm volatile("" ::: "memory");
-    if (c + NW < nsplit) load_rows(c + NW);
+    if (c + NW * S < nsplit) load_rows(c + NW * S);
 #pragma unroll
     for (int b = LPR; b < 64; b <<= 1)
 #pragma unroll
@@ -440,7 +453,12 @@ __global__ __launch_bounds__(768) void attn_head_d_kernel(const _Float16* qkv, c
       ll += wl[ww] * f;
       o += wo[ww][tid] * f;
     }
-    out[h * D + tid] = (_Float16)(o / ll);
+    if constexpr (PARTS) {
+      parts[(h * S + sp) * D + tid] = o;
+      if (tid == 0) *(float2*)(parts + (size_t)H * S * D + 2 * (h * S + sp)) = make_float2(mm, ll);
+    } else {
+      out[h * D + tid] = (_Float16)(o / ll);
+    }
   }
 }
 
@@ -584,13 +602,41 @@ hipError_t attn_fused_launch(const void* qkv, const float* cos_t, const float* s
                              void* vc, void* out, int H, int KVH, int D, int64_t L, float scale, hipStream_t s) {
   const int NW = std::min<int64_t>(12, (L + 4095 / D) / (4096 / D));   // one wave per step up to 12
   if (D == 128)
-    hipLaunchKernelGGL(attn_head_d_kernel<128>, dim3(H), dim3(64 * NW), 0, s, (const _Float16*)qkv, cos_t, sin_t,
-                       pos, (_Float16*)kc, (_Float16*)vc, (_Float16*)out, H, KVH, L, scale);
+    hipLaunchKernelGGL((attn_head_d_kernel<128, false>), dim3(H), dim3(64 * NW), 0, s, (const _Float16*)qkv, cos_t, sin_t,
+                       pos, (_Float16*)kc, (_Float16*)vc, (_Float16*)out, nullptr, H, KVH, L, scale);
   else if (D == 64)
-    hipLaunchKernelGGL(attn_head_d_kernel<64>, dim3(H), dim3(64 * NW), 0, s, (const _Float16*)qkv, cos_t, sin_t,
-                       pos, (_Float16*)kc, (_Float16*)vc, (_Float16*)out, H, KVH, L, scale);
+    hipLaunchKernelGGL((attn_head_d_kernel<64, false>), dim3(H), dim3(64 * NW), 0, s, (const _Float16*)qkv, cos_t, sin_t,
+                       pos, (_Float16*)kc, (_Float16*)vc, (_Float16*)out, nullptr, H, KVH, L, scale);
   else
     return hipErrorInvalidValue;
+  return hipGetLastError();
+}
+
+// One workgroup per head is bound by its own chain (28 heads on 256 compute
+// units): 9.75 us at 28 heads of 128 and 512 positions, 41 us at 4000.  Over
+// four, with the combine in the o_proj's staging, the pair with o_proj
+// (3584 x 3584) takes 15.8 -> 13.5 us and 47.5 -> 21.8 us, and as long as
+// before at position 30 of the same caches.  Up to 8 steps of cache one
+// workgroup already has a wave per step and the combine costs about what the
+// split saves or more: 28 heads of 128, 64 positions 11.1 -> 11.5 us; 14 heads
+// of 64, 256 positions 9.6 -> 9.9, 512 (8 steps) 10.0 -> 10.2 at position 30
+// and 10.5 -> 10.3 at 500, 576 10.1 -> 9.9 and 11.5 -> 10.3.
+bool attn_parts_supported(int H, int D, int64_t L) {
+  return (D == 64 || D == 128) && attn_fused_supported(H, D, L) && L > 8 * (4096 / D);
+}
+
+hipError_t attn_parts_launch(const void* qkv, const float* cos_t, const float* sin_t, const int64_t* pos, void* kc,
+                             void* vc, float* parts, int H, int KVH, int D, int64_t L, float scale, hipStream_t s) {
+  if (!attn_parts_supported(H, D, L)) return hipErrorInvalidValue;
+  const int64_t steps = (L + 4096 / D - 1) / (4096 / D);   // of 32 (D = 128) or 64 positions
+  const int NW = (int)std::min<int64_t>(12, (steps + kAttnParts - 1) / kAttnParts);   // one wave per step up to 12, at least 2
+  const dim3 g(H, kAttnParts), b(64 * NW);
+  if (D == 128)
+    hipLaunchKernelGGL((attn_head_d_kernel<128, true>), g, b, 0, s, (const _Float16*)qkv, cos_t, sin_t, pos,
+                       (_Float16*)kc, (_Float16*)vc, nullptr, parts, H, KVH, L, scale);
+  else
+    hipLaunchKernelGGL((attn_head_d_kernel<64, true>), g, b, 0, s, (const _Float16*)qkv, cos_t, sin_t, pos,
+                       (_Float16*)kc, (_Float16*)vc, nullptr, parts, H, KVH, L, scale);
   return hipGetLastError();
 }
 

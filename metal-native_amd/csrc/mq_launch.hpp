@@ -53,7 +53,17 @@ struct LinearArgs {
   const void* pre_weight = nullptr;
   void* pre_resid = nullptr;
   float pre_eps = 0.f;
+  // prenorm == 2: the activations are attention partials (attn_parts_launch)
+  // of K / pre_dim heads, combined while they are staged; A is not read.
+  const void* pre_parts = nullptr;
+  int pre_dim = 0;
 };
+
+// Attention over parts of the cache: per head kAttnParts partial outputs fp32
+// [head][part][D] (each the sum of exp(score - m) v), then per head and part
+// (m, sum of exp(score - m)).
+constexpr int kAttnParts = 4;
+inline size_t attn_parts_floats(int H, int D) { return (size_t)H * kAttnParts * (D + 2); }
 
 // Raise a kernel's dynamic LDS limit to `bytes` on the current device, once
 // per (kernel, device); thread-safe.
@@ -195,6 +205,11 @@ size_t attn_decode_workspace(int H, int D, int64_t L);
 bool attn_fused_supported(int H, int D, int64_t L);
 hipError_t attn_fused_launch(const void* qkv, const float* cos_t, const float* sin_t, const int64_t* pos, void* kc,
                              void* vc, void* out, int H, int KVH, int D, int64_t L, float scale, hipStream_t s);
+// the same over kAttnParts workgroups per head, leaving the partials; long
+// enough caches only
+bool attn_parts_supported(int H, int D, int64_t L);
+hipError_t attn_parts_launch(const void* qkv, const float* cos_t, const float* sin_t, const int64_t* pos, void* kc,
+                             void* vc, float* parts, int H, int KVH, int D, int64_t L, float scale, hipStream_t s);
 hipError_t attn_decode_launch(const void* q, const void* kc, const void* vc, const int64_t* pos, void* out, int H,
                               int KVH, int D, int64_t L, float scale, void* ws, hipStream_t s);
 

@@ -89,9 +89,13 @@ struct RowsKArgs {
   uint32_t sz_bytes, z_bytes;
   const _Float16* pre_delta; const _Float16* pre_weight; _Float16* pre_resid;  // fused pre-norm (PRE)
   float pre_eps;
+  // attention partials in place of A (PRE == 2): see attn_parts_floats
+  const float* pre_parts; int pre_dshift; uint32_t pre_bytes;
 };
 
-template <int FMT, int EPI, int RPW, bool PRE, int NW, int MH>
+// PRE: 0 the activations as they are, 1 the fused residual add + RMSNorm, 2 the
+// fused combine of attention partials (M = 1 both)
+template <int FMT, int EPI, int RPW, int PRE, int NW, int MH>
 __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   constexpr int S = 16 / RPW;
   constexpr int KPL = FmtTraits<FMT>::KPL;       // k per 16-byte piece
@@ -306,9 +310,27 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   {
     u4 xv[kXB];
     u4 sv[kSB], zv[kSB];
-    u4 dv[PRE ? kXB : 1], wv[PRE ? kXB : 1];
-    x_fetch(0, xv, nxb);
-    if (PRE) {  // residual delta and norm weight pieces, same indices (M = 1: piece c at 16c bytes)
+    u4 dv[PRE == 1 ? kXB : 1], wv[PRE == 1 ? kXB : 1];
+    // PRE == 2: piece tid of the row is 8 columns of one head; its partials
+    constexpr int NP = PRE == 2 ? kAttnParts : 1;
+    u4 po[NP][2];
+    uint2 pm[NP];
+    if constexpr (PRE == 2) {
+      const rsrc_t pr = make_rsrc(p.pre_parts, p.pre_bytes);
+      const int hh = (8 * tid) >> p.pre_dshift, dim = 1 << p.pre_dshift, j = (8 * tid) & (dim - 1);
+      const uint32_t ml = (uint32_t)((p.K >> p.pre_dshift) * kAttnParts) << p.pre_dshift;   // floats before the (m, l) pairs
+#pragma unroll
+      for (int s = 0; s < kAttnParts; ++s) {
+        const uint32_t off = 8 * tid < p.K ? (uint32_t)(((hh * kAttnParts + s) << p.pre_dshift) + j) * 4u : kOob;
+        po[s][0] = bload16(pr, off);
+        po[s][1] = bload16(pr, off == kOob ? kOob : off + 16u);
+        pm[s] = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(
+                                              pr, 8 * tid < p.K ? (ml + 2u * (uint32_t)(hh * kAttnParts + s)) * 4u : kOob, 0, 0));
+      }
+    } else {
+      x_fetch(0, xv, nxb);
+    }
+    if (PRE == 1) {  // residual delta and norm weight pieces, same indices (M = 1: piece c at 16c bytes)
       const rsrc_t dr = make_rsrc(p.pre_delta, p.pre_delta ? (uint32_t)(p.K * 2) : 0u);
       const rsrc_t nr = make_rsrc(p.pre_weight, (uint32_t)(p.K * 2));
 #pragma unroll
@@ -326,11 +348,32 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
     // a deep stream issued first would hold back the start of compute.
 #pragma unroll
     for (int d = 0; d < kPre; ++d) raw[d] = wload();
+    if constexpr (PRE == 2) {
+      // the parts' outputs, rescaled to the largest of their maxima, over
+      // the sum of their weights; one fp16 rounding
+      float mm = -INFINITY, ll = 0.f, o[8] = {};
 #pragma unroll
-    for (int e = 0; e < kXB; ++e) asm volatile("" : "+v"(xv[e]));
+      for (int s = 0; s < kAttnParts; ++s) {
+        asm volatile("" : "+v"(po[s][0]), "+v"(po[s][1]), "+v"(pm[s].x), "+v"(pm[s].y));
+        mm = fmaxf(mm, __uint_as_float(pm[s].x));
+      }
+#pragma unroll
+      for (int s = 0; s < kAttnParts; ++s) {
+        const float m = __uint_as_float(pm[s].x), f = m == -INFINITY ? 0.f : expf(m - mm);
+        ll += __uint_as_float(pm[s].y) * f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) o[k] += __uint_as_float(po[s][k >> 2][k & 3]) * f;
+      }
+      h8 v;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = 8 * tid < p.K ? (_Float16)(o[k] / ll) : (_Float16)0.f;
+      xv[0] = __builtin_bit_cast(u4, v);
+    }
+#pragma unroll
+    for (int e = 0; e < (PRE == 2 ? 1 : kXB); ++e) asm volatile("" : "+v"(xv[e]));
 #pragma unroll
     for (int e = 0; e < kSB; ++e) asm volatile("" : "+v"(sv[e]), "+v"(zv[e]));
-    if (PRE) {
+    if (PRE == 1) {
       // A' = half(A + delta) (the residual, stored by workgroup 0), then the
       // row's sum of squares across the workgroup, then the normalised pieces
       float ss = 0.f;
@@ -639,7 +682,7 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   }
 }
 
-template <int FMT, int EPI, int RPW, bool PRE, int NW, int MH>
+template <int FMT, int EPI, int RPW, int PRE, int NW, int MH>
 hipError_t launch5(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
   auto fn = rows_kernel<FMT, EPI, RPW, PRE, NW, MH>;
   hipError_t e = allow_dynamic_lds((const void*)fn, (int)kLds);
@@ -648,7 +691,7 @@ hipError_t launch5(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int FMT, int EPI, int RPW, bool PRE>
+template <int FMT, int EPI, int RPW, int PRE>
 hipError_t launch4(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
   if constexpr (RPW == 8 && !PRE && FMT != FMT_F16) {
     if (pl.mh == 2) {   // M = 9..16 on 8-row tiles: twelve waves (the activations are large)
@@ -669,9 +712,13 @@ hipError_t launch4(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
 template <int FMT, int EPI, int RPW>
 hipError_t launch3(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
   if constexpr (FMT != FMT_F16) {
-    if (k.pre_weight) return launch4<FMT, EPI, RPW, true>(k, pl, s);
+    if (k.pre_weight) return launch4<FMT, EPI, RPW, 1>(k, pl, s);
   }
-  return launch4<FMT, EPI, RPW, false>(k, pl, s);
+  if constexpr (FMT == FMT_INT4 && EPI == EPI_NONE && RPW <= 8) {
+    if (k.pre_parts) return launch4<FMT, EPI, RPW, 2>(k, pl, s);
+  }
+  if (k.pre_parts) return hipErrorInvalidValue;
+  return launch4<FMT, EPI, RPW, 0>(k, pl, s);
 }
 
 template <int FMT, int EPI>
@@ -794,7 +841,11 @@ RowsPlan rows_plan_k(const LinearArgs& a, int num_cus, int KP) {
   off += al16((size_t)nw * 4);
   if (off > kLds) return p;
   if ((int64_t)U * nw >= ((int64_t)1 << 31)) return p;  // unit ranges in 32-bit arithmetic
-  if (a.prenorm) {  // one staging batch, whole 16-byte pieces, M = 1
+  if (a.prenorm == 2) {   // one 8-column piece per thread, each within one head
+    if (a.M != 1 || a.fmt != FMT_INT4 || a.epi != EPI_NONE || rpw > 8 || KS * kstep / 8 > 64 * nw ||
+        (a.pre_dim != 64 && a.pre_dim != 128) || a.K % a.pre_dim || !a.pre_parts || ((uintptr_t)a.pre_parts & 15))
+      return p;
+  } else if (a.prenorm) {  // one staging batch, whole 16-byte pieces, M = 1
     const int64_t pieces = (int64_t)KS * kstep / 8;
     if (a.M != 1 || !quant || a.K % 8 || pieces > (int64_t)kXB * 64 * nw || !a.pre_weight || !a.pre_resid) return p;
     if (((uintptr_t)a.pre_weight | (uintptr_t)a.pre_resid | (uintptr_t)a.pre_delta) & 15) return p;
@@ -841,7 +892,11 @@ hipError_t rows_launch(const LinearArgs& a, const RowsPlan& pl, void* ws, hipStr
   }
   k.R = pl.R; k.TW = pl.TW; k.KS = pl.KS; k.XS = pl.XS; k.maxT = pl.maxT; k.snp = pl.snp;
   k.off_sz = pl.off_sz; k.off_scr = pl.off_scr; k.off_slot = pl.off_slot; k.off_wft = pl.off_wft;
-  if (a.prenorm) {
+  if (a.prenorm == 2) {
+    k.pre_parts = (const float*)a.pre_parts;
+    k.pre_dshift = __builtin_ctz((unsigned)a.pre_dim);
+    k.pre_bytes = (uint32_t)(attn_parts_floats(a.K / a.pre_dim, a.pre_dim) * 4);
+  } else if (a.prenorm) {
     k.pre_delta = (const _Float16*)a.pre_delta;
     k.pre_weight = (const _Float16*)a.pre_weight;
     k.pre_resid = (_Float16*)a.pre_resid;

@@ -164,9 +164,9 @@ class SyntheticDecoder:
                                              epilogue="bias", bias=L["qkv"].bias)
             x = bufs[cur]
             cur ^= 1
-            a = ops.attention_decode_rope(qkv, self.cos, self.sin, pos, self.kv[li, 0], self.kv[li, 1], H, KVH, Dh,
-                                          scale)
-            act = ops.rmsnorm_dequant_matmul(x, L["o"](a), L["ln2"], cfg.eps, bufs[cur], *L["gate_up"].operands(),
+            o = ops.attention_decode_rope_linear(qkv, self.cos, self.sin, pos, self.kv[li, 0], self.kv[li, 1], H, KVH,
+                                                 Dh, scale, *L["o"].operands())
+            act = ops.rmsnorm_dequant_matmul(x, o, L["ln2"], cfg.eps, bufs[cur], *L["gate_up"].operands(),
                                              epilogue="swiglu")
             x = bufs[cur]
             cur ^= 1

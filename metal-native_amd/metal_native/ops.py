@@ -520,6 +520,35 @@ def attention_decode_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tenso
     return out
 
 
+def attention_decode_rope_linear(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
+                                 k_cache: torch.Tensor, v_cache: torch.Tensor, heads: int, kv_heads: int, head_dim: int,
+                                 scale: float, weights_packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor,
+                                 group_size: int, quant_type: str) -> torch.Tensor:
+    """``dequant_matmul(attention_decode_rope(...), ...)``, the output
+    projection: where the kernels take the shape, the attention runs on four
+    workgroups per head and the projection combines their partials while it
+    stages its activations."""
+    qt = quant_type_code(quant_type)
+    (N, cols), L, K = weights_packed.shape, k_cache.shape[1], heads * head_dim
+    if cols * (2 if quant_type == "int4" else 1) == K and _L.mq_attention_parts_supported(N, heads, head_dim, L,
+                                                                                         group_size, qt):
+        stream = _stream_handle(qkv.device)
+        parts = torch.empty(_L.mq_attention_parts_size(heads, head_dim) // 4, dtype=torch.float32, device=qkv.device)
+        _check(_L.mq_attention_decode_rope_parts_f16(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(pos), _ptr(k_cache),
+                                                     _ptr(v_cache), _ptr(parts), heads, kv_heads, head_dim, L,
+                                                     float(scale), stream))
+        out = torch.empty((1, N), dtype=torch.float16, device=qkv.device)
+        weights_packed, ldw = _rowmajor(weights_packed, "weights_packed", "dequant_matmul")
+        rc = _L.mq_attention_parts_dequant_matmul(_ptr(parts), heads, head_dim, _ptr(weights_packed), ldw,
+                                                  _ptr(scales), _ptr(zeros), _ptr(out), N, group_size, qt, stream)
+        if rc == 0:
+            return out
+        if rc != 4:   # weights aligned otherwise than the kernel needs: the attention again, in one piece
+            _check(rc)
+    a = attention_decode_rope(qkv, cos, sin, pos, k_cache, v_cache, heads, kv_heads, head_dim, scale)
+    return dequant_matmul(a, weights_packed, scales, zeros, group_size, quant_type)
+
+
 def argmax_embed_workspace(vocab: int, device) -> torch.Tensor:
     """Zeroed workspace for ``argmax_embed``; keep one per stream."""
     nb = _L.mq_argmax_embed_workspace_size(int(vocab))
