@@ -267,11 +267,11 @@ MQ_API int mq_read_probe(const void* p, int64_t bytes, void* sink, void* stream)
  * where it takes the shape --, 1 always the 16x16x32 tiled kernel, 2 the
  * register-dequant GEMM wherever it takes the shape; all compute the same
  * contract), "gemm_rows" (rows per tile of the many-row GEMM: 64, 128 or 256, 0
- * automatic) and "gemm_parts" (its K parts, 1..64, 0 automatic), both read when
- * force_path is 13, "gemm_split" (1, the default: the 32x32x16 kernels split
+ * automatic) and "gemm_parts" (its K parts, 1..64 with 64 rows, 1..16 with more,
+ * 0 automatic), both read when force_path is 13, "gemm_split" (1, the default: the 32x32x16 kernels split
  * K over several workgroups per output tile where its tiles would leave CUs
- * idle, summing the parts in a fixed order; 0: one workgroup per tile).  A forced path that cannot take the shape falls back
- * to the automatic choice.  Returns MQ_INVALID_ARGUMENT for an unknown key or
+ * idle, summing the parts in a fixed order; 0: one workgroup per tile).  A forced path that cannot take the shape, or not
+ * with these rows and parts, falls back to the automatic choice.  Returns MQ_INVALID_ARGUMENT for an unknown key or
  * value. */
 MQ_API int mq_set_option(const char* key, int64_t value);
 

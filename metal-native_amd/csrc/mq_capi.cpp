@@ -68,9 +68,10 @@ std::atomic<int> g_gemm_impl{0};
 // tiles leave CUs idle, 0 keeps one workgroup per tile
 std::atomic<int> g_gemm_split{1};
 
-// gemm_rows: rows per tile of the many-row GEMM (128 or 256), 0 automatic
+// read where force_path is PATH_GEMMN only: rows per tile of the many-row GEMM
+// (64, 128 or 256) and its K parts (1..64; at most 16 with 128 and 256 rows),
+// 0 automatic
 std::atomic<int> g_gemm_rows{0};
-// gemm_parts: K parts of the many-row GEMM (1..16), 0 automatic
 std::atomic<int> g_gemm_parts{0};
 
 mq::GemvTuning gemv_tuning() {
@@ -185,13 +186,22 @@ bool short_rows(const mq::LinearArgs& a) {
   return a.K <= 1024 || (a.fmt == mq::FMT_INT4 && a.M <= 2 && a.K <= 1536);
 }
 
-int choose_path(const mq::LinearArgs& a, bool noalloc) {
-  int forced = g_force_path.load();
+// The many-row GEMM with the rows and parts of the options; not ok where it
+// cannot take the shape, or the shape those rows and parts.
+mq::GemmnPlan gemmn_forced(const mq::LinearArgs& a, bool allow_split) {
+  return mq::gemmn_plan(a, num_cus_current(), allow_split, g_gemm_rows.load() / 32, allow_split ? g_gemm_parts.load() : 1);
+}
+
+// The path of a call; with PATH_GEMMN, *gn is its plan (of one K part where
+// allow_parts is false).  The options are read here only, so that the path
+// and the plan agree whatever another thread sets meanwhile.
+int choose_path(const mq::LinearArgs& a, bool noalloc, bool allow_parts, mq::GemmnPlan* gn) {
+  const int forced = g_force_path.load();
   if (forced == PATH_ROWS && rows_ok(a)) return PATH_ROWS;
   if (forced == PATH_RSTREAM && mq::rstream_plan(a, num_cus_current()).ok) return PATH_RSTREAM;
   if (forced == PATH_DECODE && decode_ok(a)) return PATH_DECODE;
   if (forced == PATH_TILED && prefill_ok(a)) return PATH_TILED;
-  if (forced == PATH_GEMMN && mq::gemmn_supported(a)) return PATH_GEMMN;
+  if (forced == PATH_GEMMN && (*gn = gemmn_forced(a, allow_parts)).ok) return PATH_GEMMN;
   if (forced == PATH_GENERIC) return PATH_GENERIC;
   // automatic choice: the row-block kernel up to M = 4; for M = 5..16 only
   // where the activations fit in LDS whole (its K parts measured slower than
@@ -211,7 +221,7 @@ int choose_path(const mq::LinearArgs& a, bool noalloc) {
   // on 13 shapes, e.g. config 2 at M = 9 / 16: 19.0-19.7 / 21.6 us against
   // 25.0 / 25.4 us, K = 4096, N = 4096, M = 16: 8.3 against 12.0 us)
   if (a.M >= 5 && a.M <= 16 && mq::rstream_plan(a, num_cus_current()).ok) return PATH_RSTREAM;
-  if (gemmn_auto(a, !noalloc).ok) return PATH_GEMMN;
+  if ((*gn = gemmn_auto(a, allow_parts)).ok) return PATH_GEMMN;
   // M = 9..16 with long rows the register-streamed plan declines: the prefill GEMM with K split over
   // workgroups beats the split-K GEMV (measured at K >= 8192 on 6 shapes at
   // M = 9, 12, 13-16: faster on all but K = 8192, N = 4096 (2-10 % slower
@@ -228,8 +238,20 @@ int choose_path(const mq::LinearArgs& a, bool noalloc) {
 // noalloc: the split-K GEMV uses the library's fixed scratch array instead of
 // the per-stream workspace (no allocation on any path).
 int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
-  int path = choose_path(a, noalloc);
+  mq::GemmnPlan gn{};
+  int path = choose_path(a, noalloc, !noalloc, &gn);
   hipError_t e = hipSuccess;
+  void* gn_ws = nullptr;
+  if (path == PATH_GEMMN) {
+    e = workspace_for(s, gn.ws_bytes, &gn_ws);
+    if (e == hipErrorStreamCaptureUnsupported) {
+      // under capture with a workspace too small for this plan: the choice
+      // among the kernels that need none
+      path = choose_path(a, noalloc, false, &gn);
+      e = hipSuccess;
+    }
+    if (e != hipSuccess) return hip_fail(e, "dequant_matmul: workspace allocation failed");
+  }
   if (path == PATH_ROWS) {
     // K parts need the workspace: the no-allocation entry point takes the
     // split-K GEMV (whose scratch is fixed) for such shapes
@@ -247,28 +269,11 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
     }
   }
   if (path == PATH_GEMMN) {
-    const int rows = g_gemm_rows.load(), parts = g_gemm_parts.load();
-    auto planned = [&](bool split) {
-      return g_force_path.load() == PATH_GEMMN ? mq::gemmn_plan(a, num_cus_current(), split, rows / 32, split ? parts : 1)
-                                               : gemmn_auto(a, split);
-    };
-    mq::GemmnPlan pl = planned(!noalloc);
-    void* ws = nullptr;
-    e = workspace_for(s, pl.ws_bytes, &ws);
-    if (e == hipErrorStreamCaptureUnsupported) {
-      // under capture with a workspace too small for this shape: the choice
-      // among the kernels that need none
-      e = hipSuccess;
-      pl = planned(false);
-      if (!pl.ok) path = PATH_TILED;
-    }
-    if (e != hipSuccess) return hip_fail(e, "dequant_matmul: workspace allocation failed");
-    if (pl.ok) e = mq::gemmn_launch(a, pl, ws, s);
-  }
-  if (path == PATH_RSTREAM) {
+    e = mq::gemmn_launch(a, gn, gn_ws, s);
+  } else if (path == PATH_RSTREAM) {
     const mq::RsPlan pl = mq::rstream_plan(a, num_cus_current());
     e = pl.ok ? mq::rstream_launch(a, pl, s) : hipErrorInvalidValue;
-  } else if (path == PATH_ROWS || path == PATH_GEMMN) {
+  } else if (path == PATH_ROWS) {
   } else if (path == PATH_DECODE) {
     const mq::GemvPlan pl = mq::gemv_plan(a, num_cus_current(), gemv_tuning());
     void* ws = nullptr;
@@ -572,7 +577,8 @@ MQ_API int mq_vecmat_f16(const void* a, int64_t lda, const void* b, int64_t ldb,
   la.g = 1; la.G = 1;
   la.fmt = mq::FMT_F16;
   la.epi = mq::EPI_NONE;
-  const int pth = choose_path(la, false);
+  mq::GemmnPlan gn{};
+  const int pth = choose_path(la, false, true, &gn);
   if (pth == PATH_DECODE || pth == PATH_ROWS) return run_linear(la, (hipStream_t)stream);
   hipError_t e = mq::generic_linear_launch(la, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "matmul: kernel launch failed");

@@ -184,6 +184,24 @@ def test_one_hot_selects_dequantized_weights(mn, gpu, rows, qt, mixed):
             assert not bad.any(), f"{bad.sum()} differ, e.g. {y[bad][:4]} vs {want[:, ks].T[bad][:4]}"
 
 
+@pytest.mark.parametrize("rows,parts,M,K,N", [
+    (256, 32, 300, 2048, 514),     # more parts than that tile height takes
+    (128, 17, 130, 1088, 256),
+    (128, 16, 2048, 1024, 8192),   # partial sums beyond the bound on the workspace
+])
+def test_forced_plan_the_kernel_declines(mn, gpu, rows, parts, M, K, N):
+    """Rows and parts that the kernel does not take: the automatic choice
+    runs and writes every output."""
+    x, wp, s, z, g, acc = problem(M, K, N, 64, "int4", seed=parts)
+    out = torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu)
+    args = dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, "int4"
+    with forced(mn, rows, parts):
+        mn.dequant_matmul(*args, out=out)
+        path = mn.last_path()
+    check(out.cpu().numpy(), acc, what=path)
+    assert torch.equal(mn.dequant_matmul(*args), out) and mn.last_path() == path
+
+
 @pytest.mark.parametrize("M,K,N,g,qt,epi,want", [
     (777, 4096, 3584, 128, "int4", "swiglu", "gemmn"),
     (300, 8192, 2048, 32, "int4", None, "gemmn"),       # K parts; more groups than the other kernels' tables hold
