@@ -60,12 +60,19 @@ def _compile(src: str, hipcc: str) -> str:
 
 
 def _compile_front() -> str:
-    """The object of csrc/mq_torch.cpp: host code against torch's headers."""
+    """The object of csrc/mq_torch.cpp: host code against torch's headers.
+
+    NDEBUG leaves out pybind11's per-thread reference counter, the front's only
+    thread-local variable: a library with thread-local storage that is loaded
+    late puts every thread-local access of the process (each torch call makes
+    several) on the loader's slow path until the thread touches that library's
+    own, which nothing here would do.  quantize + dequantize of a small layer
+    after another call: 26.8 us with the counter, 24.1 without."""
     import torch  # noqa: PLC0415
 
     inc = os.path.join(os.path.dirname(torch.__file__), "include")
     obj = os.path.join(BUILD_DIR, "mq_torch.o")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden",
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-DNDEBUG",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            f"-I{inc}", f"-I{os.path.join(inc, 'torch', 'csrc', 'api', 'include')}",
            f"-I{sysconfig.get_paths()['include']}", "-c", os.path.join(CSRC, "mq_torch.cpp"), "-o", obj]

@@ -25,6 +25,25 @@ def test_declines_what_is_not_a_plain_gpu_tensor(mn):
         mn.dequant_matmul(x, w, s, s, 32, "int4")
 
 
+def test_front_has_no_thread_local_storage(mn):
+    """No PT_TLS segment: loading one late slows every thread-local access of
+    the importing thread (glibc's stale thread vector) until that thread
+    touches the newest library's own variables."""
+    import struct
+
+    from metal_native import _mq_torch
+
+    with open(_mq_torch.__file__, "rb") as f:
+        head = f.read(64)
+        assert head[:6] == b"\x7fELF\x02\x01"
+        (phoff,) = struct.unpack_from("<Q", head, 32)
+        size, count = struct.unpack_from("<HH", head, 54)
+        f.seek(phoff)
+        table = f.read(size * count)
+    types = [struct.unpack_from("<I", table, size * i)[0] for i in range(count)]
+    assert 1 in types and 7 not in types   # PT_LOAD, PT_TLS
+
+
 class Marked(torch.Tensor):
     pass
 
