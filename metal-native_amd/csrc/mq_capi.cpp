@@ -87,16 +87,21 @@ bool decode_ok(const mq::LinearArgs& a) {
 
 // Split-K workspace, one per (device, stream): counters must start at zero and
 // every launch leaves them at zero, so one fill at allocation suffices.
-// Calls on one stream are ordered, so they may share it.
+// Calls on one stream are ordered, so they may share it; mu is held from the
+// first to the last launch of a call that uses it, so that no other thread's
+// call on the stream comes between them (a many-row GEMM of several K parts
+// is two launches: the parts, and their sum).
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
+  std::mutex mu;
 };
 std::mutex g_ws_mu;
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 std::vector<void*> g_ws_retired;   // superseded workspaces: kept until the process ends
 
-hipError_t workspace_for(hipStream_t s, size_t need, void** out) {
+// `hold` locks the workspace where one is given out.
+hipError_t workspace_for(hipStream_t s, size_t need, void** out, std::unique_lock<std::mutex>& hold) {
   *out = nullptr;
   if (need == 0) return hipSuccess;
   int dev = 0;
@@ -104,6 +109,7 @@ hipError_t workspace_for(hipStream_t s, size_t need, void** out) {
   if (e != hipSuccess) return e;
   std::lock_guard<std::mutex> lk(g_ws_mu);
   Workspace& w = g_ws[{dev, s}];
+  std::unique_lock<std::mutex> in_use(w.mu);
   if (w.bytes < need) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
@@ -126,6 +132,7 @@ hipError_t workspace_for(hipStream_t s, size_t need, void** out) {
     w.bytes = nb;
   }
   *out = w.ptr;
+  hold = std::move(in_use);
   return hipSuccess;
 }
 
@@ -241,9 +248,10 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
   mq::GemmnPlan gn{};
   int path = choose_path(a, noalloc, !noalloc, &gn);
   hipError_t e = hipSuccess;
+  std::unique_lock<std::mutex> hold;   // of the workspace, until the call's last launch
   void* gn_ws = nullptr;
   if (path == PATH_GEMMN) {
-    e = workspace_for(s, gn.ws_bytes, &gn_ws);
+    e = workspace_for(s, gn.ws_bytes, &gn_ws, hold);
     if (e == hipErrorStreamCaptureUnsupported) {
       // under capture with a workspace too small for this plan: the choice
       // among the kernels that need none
@@ -258,7 +266,7 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
     const mq::RowsPlan pl = mq::rows_plan(a, num_cus_current(), !noalloc);
     if (pl.ok) {
       void* ws = nullptr;
-      e = workspace_for(s, pl.ws_bytes, &ws);
+      e = workspace_for(s, pl.ws_bytes, &ws, hold);
       if (e == hipErrorStreamCaptureUnsupported)
         return fail(MQ_INVALID_ARGUMENT, "dequant_matmul: the split-K workspace of this stream is too small; "
                                          "make one call of this shape on the stream before capturing it");
@@ -287,7 +295,7 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
         if (e != hipSuccess) return hip_fail(e, "dequant_matmul_noalloc: scratch set-up failed");
       }
     } else {
-      e = workspace_for(s, pl.ws_bytes, &ws);
+      e = workspace_for(s, pl.ws_bytes, &ws, hold);
       if (e == hipErrorStreamCaptureUnsupported && a.M <= 4 && rows_ok(a)) {
         // under capture with a workspace too small for this shape: the
         // row-block kernel in one part (no workspace) rather than an error
@@ -315,7 +323,7 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
       bool split = !noalloc && g_gemm_split.load() != 0;
       void* ws = nullptr;
       size_t need = split ? mq::gemmw_ws_bytes(a, cus, true) : 0;
-      hipError_t we = workspace_for(s, need, &ws);
+      hipError_t we = workspace_for(s, need, &ws, hold);
       if (we == hipErrorStreamCaptureUnsupported) {
         // under capture with a workspace too small for this shape: one
         // workgroup per tile (no workspace) rather than an error

@@ -248,3 +248,37 @@ def test_capture_and_shared_workspace(mn, gpu):
                 got = mn.dequant_matmul(*vargs)
             torch.cuda.synchronize()
             check(got.cpu().numpy(), vref, what="split-K GEMV between replays")
+
+
+def test_threads_on_one_stream(mn, gpu):
+    """Calls of several K parts (two launches that share the stream's
+    workspace) from threads on one stream, among calls of the split-K GEMV on
+    the same workspace: each gives what it gives alone."""
+    import threading
+
+    shapes = [(300, 8192, 2048, 128, "gemmn"), (130, 8192, 1024, 128, "gemmn"), (8, 8192, 3072, 128, None),
+              (37, 18944, 512, 128, "gemmn")]
+    calls, want = [], []
+    for i, (M, K, N, g, path) in enumerate(shapes):
+        args = tuple(dev(a, gpu) for a in O.make_int4_problem(M, K, N, g, seed=60 + i)) + (g, "int4")
+        want.append(mn.dequant_matmul(*args))
+        assert path is None or mn.last_path() == path
+        calls.append(args)
+    got = [[] for _ in shapes]
+    start = threading.Barrier(len(shapes))
+
+    def work(i):
+        start.wait()
+        for _ in range(150):
+            got[i].append(mn.dequant_matmul(*calls[i]))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(shapes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for i, outs in enumerate(got):
+        assert len(outs) == 150
+        wrong = sum(not torch.equal(y, want[i]) for y in outs)
+        assert not wrong, f"{wrong} of {len(outs)} calls of {shapes[i]} differ"
