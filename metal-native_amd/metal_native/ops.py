@@ -107,6 +107,41 @@ def quant_type_code(quant_type: str) -> int:
     return _lib.QUANT_INT4 if quant_type == "int4" else _lib.QUANT_INT8
 
 
+def _check_weight_operands(op: str, K: int, device: torch.device, weights_packed: torch.Tensor, scales: torch.Tensor,
+                           zeros: torch.Tensor, group_size: int, quant_type: str) -> int:
+    """Type, shape and device checks of a quantized weight for activations of
+    ``K`` columns on ``device``; returns the quantization type's code."""
+    if group_size not in (32, 64, 128) and group_size != K:
+        _invalid("dequant_matmul: group_size must be 32, 64, or 128")
+    qt = quant_type_code(quant_type)
+    for t, what in ((weights_packed, "weights_packed"), (scales, "scales"), (zeros, "zeros")):
+        _require_cuda(t, what, op)
+        if t.device != device:
+            _invalid(f"{op}: {what} must be on the activations' device")
+    if weights_packed.dim() != 2:
+        _invalid(f"{op}: weights_packed must be 2D")
+    N = weights_packed.shape[0]
+    if qt == _lib.QUANT_INT4:
+        if weights_packed.shape[1] != K // 2:
+            _invalid("dequant_matmul: INT4 weights must be [N, K/2]")
+        if K % 2:
+            _invalid("dequant_matmul: INT4 weights must be [N, K/2] with K even")
+        if weights_packed.dtype not in (torch.uint8, torch.int8):
+            _invalid(f"{op}: INT4 weights must be uint8 (two nibbles per byte)")
+    else:
+        if weights_packed.shape[1] != K:
+            _invalid("dequant_matmul: INT8 weights must be [N, K]")
+        if weights_packed.dtype not in (torch.int8, torch.uint8):
+            _invalid(f"{op}: INT8 weights must be int8")
+    G = (K + group_size - 1) // group_size
+    for t, what in ((scales, "scales"), (zeros, "zeros")):
+        if t.dtype != torch.float16:
+            _invalid(f"{op}: {what} must be Float16")
+        if tuple(t.shape) != (N, G):
+            _invalid(f"{op}: {what} must be [N, ceil(K/group_size)] = [{N}, {G}], got {list(t.shape)}")
+    return qt
+
+
 def dequant_matmul(activations: torch.Tensor, weights_packed: torch.Tensor, scales: torch.Tensor,
                    zeros: torch.Tensor, group_size: int, quant_type: str, *,
                    epilogue: str | None = None, bias: torch.Tensor | None = None,
@@ -142,34 +177,8 @@ def dequant_matmul(activations: torch.Tensor, weights_packed: torch.Tensor, scal
     if activations.dtype != torch.float16:
         _invalid("dequant_matmul: activations must be Float16")
     M, K = activations.shape
-    if group_size not in (32, 64, 128) and group_size != K:
-        _invalid("dequant_matmul: group_size must be 32, 64, or 128")
-    qt = quant_type_code(quant_type)
-    for t, what in ((weights_packed, "weights_packed"), (scales, "scales"), (zeros, "zeros")):
-        _require_cuda(t, what, op)
-        if t.device != activations.device:
-            _invalid(f"{op}: {what} must be on the activations' device")
-    if weights_packed.dim() != 2:
-        _invalid(f"{op}: weights_packed must be 2D")
+    qt = _check_weight_operands(op, K, activations.device, weights_packed, scales, zeros, group_size, quant_type)
     N = weights_packed.shape[0]
-    if qt == _lib.QUANT_INT4:
-        if weights_packed.shape[1] != K // 2:
-            _invalid("dequant_matmul: INT4 weights must be [N, K/2]")
-        if K % 2:
-            _invalid("dequant_matmul: INT4 weights must be [N, K/2] with K even")
-        if weights_packed.dtype not in (torch.uint8, torch.int8):
-            _invalid(f"{op}: INT4 weights must be uint8 (two nibbles per byte)")
-    else:
-        if weights_packed.shape[1] != K:
-            _invalid("dequant_matmul: INT8 weights must be [N, K]")
-        if weights_packed.dtype not in (torch.int8, torch.uint8):
-            _invalid(f"{op}: INT8 weights must be int8")
-    G = (K + group_size - 1) // group_size
-    for t, what in ((scales, "scales"), (zeros, "zeros")):
-        if t.dtype != torch.float16:
-            _invalid(f"{op}: {what} must be Float16")
-        if tuple(t.shape) != (N, G):
-            _invalid(f"{op}: {what} must be [N, ceil(K/group_size)] = [{N}, {G}], got {list(t.shape)}")
     if epilogue not in _EPILOGUES:
         _invalid(f"{op}: unknown epilogue {epilogue!r}")
     epi = _EPILOGUES[epilogue]
@@ -528,23 +537,27 @@ def attention_decode_rope_linear(qkv: torch.Tensor, cos: torch.Tensor, sin: torc
     projection: where the kernels take the shape, the attention runs on four
     workgroups per head and the projection combines their partials while it
     stages its activations."""
-    qt = quant_type_code(quant_type)
-    (N, cols), L, K = weights_packed.shape, k_cache.shape[1], heads * head_dim
-    if cols * (2 if quant_type == "int4" else 1) == K and _L.mq_attention_parts_supported(N, heads, head_dim, L,
-                                                                                         group_size, qt):
-        stream = _stream_handle(qkv.device)
-        parts = torch.empty(_L.mq_attention_parts_size(heads, head_dim) // 4, dtype=torch.float32, device=qkv.device)
-        _check(_L.mq_attention_decode_rope_parts_f16(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(pos), _ptr(k_cache),
-                                                     _ptr(v_cache), _ptr(parts), heads, kv_heads, head_dim, L,
-                                                     float(scale), stream))
-        out = torch.empty((1, N), dtype=torch.float16, device=qkv.device)
-        weights_packed, ldw = _rowmajor(weights_packed, "weights_packed", "dequant_matmul")
-        rc = _L.mq_attention_parts_dequant_matmul(_ptr(parts), heads, head_dim, _ptr(weights_packed), ldw,
-                                                  _ptr(scales), _ptr(zeros), _ptr(out), N, group_size, qt, stream)
-        if rc == 0:
-            return out
-        if rc != 4:   # weights aligned otherwise than the kernel needs: the attention again, in one piece
-            _check(rc)
+    K, L = heads * head_dim, k_cache.shape[1]
+    dev = qkv.device
+    qt = _check_weight_operands("dequant_matmul", K, dev, weights_packed, scales, zeros, group_size, quant_type)
+    weights_packed, ldw = _rowmajor(weights_packed, "weights_packed", "dequant_matmul")
+    N, cols = weights_packed.shape
+    # the plan that mq_attention_parts_supported answers for: rows without gaps, 16-byte aligned
+    if ldw == cols and weights_packed.data_ptr() % 16 == 0 and _L.mq_attention_parts_supported(N, heads, head_dim, L,
+                                                                                               group_size, qt):
+        scales = scales.contiguous()
+        zeros = zeros.contiguous()
+        parts = torch.empty(_L.mq_attention_parts_size(heads, head_dim) // 4, dtype=torch.float32, device=dev)
+        out = torch.empty((1, N), dtype=torch.float16, device=dev)
+        with torch.cuda.device(dev):
+            stream = _stream_handle(dev)
+            _check(_L.mq_attention_decode_rope_parts_f16(_ptr(qkv), _ptr(cos), _ptr(sin), _ptr(pos), _ptr(k_cache),
+                                                         _ptr(v_cache), _ptr(parts), heads, kv_heads, head_dim, L,
+                                                         float(scale), stream))
+            _check(_L.mq_attention_parts_dequant_matmul(_ptr(parts), heads, head_dim, _ptr(weights_packed), ldw,
+                                                        _ptr(scales), _ptr(zeros), _ptr(out), N, group_size, qt,
+                                                        stream))
+        return out
     a = attention_decode_rope(qkv, cos, sin, pos, k_cache, v_cache, heads, kv_heads, head_dim, scale)
     return dequant_matmul(a, weights_packed, scales, zeros, group_size, quant_type)
 

@@ -62,6 +62,67 @@ def test_matches_one_workgroup_per_head(gpu, H, KVH, D, L, N, where):
     assert bool(((got.double() - want.double()).abs().cpu() <= bound).all())
 
 
+def _wider(t, by=16):
+    big = torch.full((t.shape[0], t.shape[1] + by), 77, dtype=t.dtype, device=t.device)
+    big[:, :t.shape[1]] = t
+    return big[:, :t.shape[1]]
+
+
+def _shifted(t):
+    """The same matrix at an address that is not 16-byte aligned."""
+    flat = torch.empty(t.numel() + 2, dtype=t.dtype, device=t.device)[2:]
+    return flat.copy_(t.flatten()).view(t.shape)
+
+
+@pytest.mark.parametrize("L", [576, 64])   # with and without the four-workgroup attention
+@pytest.mark.parametrize("form", ["weights", "scales", "zeros", "columns strided", "weights shifted", "scales shifted",
+                                  "rows expanded"])
+def test_operands_of_every_layout(gpu, L, form):
+    """Operands that are not contiguous or not aligned give what contiguous ones give."""
+    from metal_native import ops
+
+    H, KVH, D, N = 8, 2, 128, 640
+    cos, sin, kc, vc, qkv, o = _case(gpu, H, KVH, D, L, N, seed=11)
+    w, s, z, g, qt = o.operands()
+    if form == "rows expanded":
+        w, s, z = (t[:1].expand(t.shape) for t in (w, s, z))
+    p, scale = torch.tensor([50], device=gpu), 1.0 / math.sqrt(D)
+    a = ops.attention_decode_rope(qkv, cos, sin, p, kc, vc, H, KVH, D, scale)
+    want = ops.attention_decode_rope_linear(qkv, cos, sin, p, kc, vc, H, KVH, D, scale, w.contiguous(), s.contiguous(),
+                                            z.contiguous(), g, qt)
+    # (the bound of two attentions that differ in fp32 order, in the loosest form that a wrong operand fails)
+    assert float((want - ops.dequant_matmul(a, w, s, z, g, qt)).double().norm() / want.double().norm()) < 1e-2
+    change = {"weights": (_wider, "w"), "scales": (_wider, "s"), "zeros": (_wider, "z"),
+              "columns strided": (lambda t: torch.stack((t, t), -1)[..., 0], "wsz"), "weights shifted": (_shifted, "w"),
+              "scales shifted": (_shifted, "sz"), "rows expanded": (lambda t: t, "")}[form]
+    w, s, z = (change[0](t) if n in change[1] else t for n, t in zip("wsz", (w, s, z)))
+    got = ops.attention_decode_rope_linear(qkv, cos, sin, p, kc, vc, H, KVH, D, scale, w, s, z, g, qt)
+    if form in ("weights", "weights shifted"):   # the two calls, on another kernel: rows with gaps or not aligned
+        assert torch.equal(got, ops.dequant_matmul(a, w, s, z, g, qt))
+    else:
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("L", [576, 64])
+def test_refuses_what_dequant_matmul_refuses(gpu, L):
+    import metal_native as mn
+    from metal_native import ops
+
+    H, KVH, D, N = 8, 2, 128, 640
+    cos, sin, kc, vc, qkv, o = _case(gpu, H, KVH, D, L, N, seed=12)
+    w, s, z, g, qt = o.operands()
+    p = torch.tensor([50], device=gpu)
+    before = kc.clone(), vc.clone()
+    for args, match in [((w, s[:, 1:].contiguous(), z, g, qt), "scales must be"), ((w, s, z[:-1], g, qt), "zeros must be"),
+                        ((w, s.float(), z, g, qt), "scales must be Float16"), ((w, s, None, g, qt), "zeros must be"),
+                        ((w, s.cpu(), z, g, qt), "scales must be a GPU tensor"), ((w.half(), s, z, g, qt), "uint8"),
+                        ((w[:, 1:], s, z, g, qt), "INT4 weights"), ((w, s, z, 48, qt), "group_size"),
+                        ((w, s, z, g, "int8"), "INT8 weights"), ((w.flatten(), s, z, g, qt), "2D")]:
+        with pytest.raises(mn.MetalNativeError, match=match):
+            ops.attention_decode_rope_linear(qkv, cos, sin, p, kc, vc, H, KVH, D, 1.0, *args)
+    assert torch.equal(kc, before[0]) and torch.equal(vc, before[1])
+
+
 def test_error_against_float64_no_larger(gpu):
     """The error of the split attention + projection over the ranges of the
     decode step, against float64 from the same fp16 operands."""
