@@ -165,7 +165,7 @@ class SyntheticDecoder:
             x = bufs[cur]
             cur ^= 1
             o = ops.attention_decode_rope_linear(qkv, self.cos, self.sin, pos, self.kv[li, 0], self.kv[li, 1], H, KVH,
-                                                 Dh, scale, *L["o"].operands())
+                                                 Dh, scale, *L["o"].operands(), bias=L["o"].bias)
             act = ops.rmsnorm_dequant_matmul(x, o, L["ln2"], cfg.eps, bufs[cur], *L["gate_up"].operands(),
                                              epilogue="swiglu")
             x = bufs[cur]
@@ -202,8 +202,10 @@ class SyntheticDecoder:
         dev = self.device
         def lin(ql, x, name="", li=-1):
             y = x.float() @ dequant(ql).to(dev).float().t()
+            if ql.bias is not None:
+                y = y + ql.bias.float()
             if probe is not None:
-                probe(name, li, ql, x, y + (ql.bias.float() if name == "qkv" else 0.0))
+                probe(name, li, ql, x, y)
             return y
 
         x = self.embed[token:token + 1]
@@ -212,7 +214,7 @@ class SyntheticDecoder:
         kv = self.kv.clone()
         for li, L in enumerate(self.layers):
             h = rms_norm(x, L["ln1"], cfg.eps)
-            qkv = (lin(L["qkv"], h, "qkv", li) + L["qkv"].bias.float()).half()[0]
+            qkv = lin(L["qkv"], h, "qkv", li).half()[0]
             q = apply_rope(qkv[:H * Dh].view(H, Dh), cos, sin)
             k = apply_rope(qkv[H * Dh:(H + KVH) * Dh].view(KVH, Dh), cos, sin)
             v = qkv[(H + KVH) * Dh:].view(KVH, Dh)

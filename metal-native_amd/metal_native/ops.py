@@ -532,19 +532,20 @@ def attention_decode_rope(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tenso
 def attention_decode_rope_linear(qkv: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, pos: torch.Tensor,
                                  k_cache: torch.Tensor, v_cache: torch.Tensor, heads: int, kv_heads: int, head_dim: int,
                                  scale: float, weights_packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor,
-                                 group_size: int, quant_type: str) -> torch.Tensor:
+                                 group_size: int, quant_type: str, *, bias: torch.Tensor | None = None) -> torch.Tensor:
     """``dequant_matmul(attention_decode_rope(...), ...)``, the output
-    projection: where the kernels take the shape, the attention runs on four
-    workgroups per head and the projection combines their partials while it
-    stages its activations."""
+    projection, with a ``bias`` added where one is given: where the kernels
+    take the shape and there is no bias, the attention runs on four workgroups
+    per head and the projection combines their partials while it stages its
+    activations."""
     K, L = heads * head_dim, k_cache.shape[1]
     dev = qkv.device
     qt = _check_weight_operands("dequant_matmul", K, dev, weights_packed, scales, zeros, group_size, quant_type)
     weights_packed, ldw = _rowmajor(weights_packed, "weights_packed", "dequant_matmul")
     N, cols = weights_packed.shape
     # the plan that mq_attention_parts_supported answers for: rows without gaps, 16-byte aligned
-    if ldw == cols and weights_packed.data_ptr() % 16 == 0 and _L.mq_attention_parts_supported(N, heads, head_dim, L,
-                                                                                               group_size, qt):
+    if (bias is None and ldw == cols and weights_packed.data_ptr() % 16 == 0
+            and _L.mq_attention_parts_supported(N, heads, head_dim, L, group_size, qt)):
         scales = scales.contiguous()
         zeros = zeros.contiguous()
         parts = torch.empty(_L.mq_attention_parts_size(heads, head_dim) // 4, dtype=torch.float32, device=dev)
@@ -559,7 +560,8 @@ def attention_decode_rope_linear(qkv: torch.Tensor, cos: torch.Tensor, sin: torc
                                                         stream))
         return out
     a = attention_decode_rope(qkv, cos, sin, pos, k_cache, v_cache, heads, kv_heads, head_dim, scale)
-    return dequant_matmul(a, weights_packed, scales, zeros, group_size, quant_type)
+    return dequant_matmul(a, weights_packed, scales, zeros, group_size, quant_type,
+                          epilogue=None if bias is None else "bias", bias=bias)
 
 
 def argmax_embed_workspace(vocab: int, device) -> torch.Tensor:

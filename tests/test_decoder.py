@@ -47,6 +47,27 @@ def test_decode_step_matches_oracle_reference(gpu):
         assert int(nxt.item()) == int(torch.argmax(ref).item())
 
 
+@pytest.mark.parametrize("max_len", [32, 600])   # attention on one and on four workgroups per head
+def test_bias_of_the_output_projection(gpu, max_len):
+    from dataclasses import replace
+
+    from metal_native.decoder import SyntheticDecoder
+
+    m = SyntheticDecoder(replace(tiny(), max_len=max_len), gpu, seed=3, prefilled=16)
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(1)
+    for layer in m.layers:
+        layer["o"].bias = (torch.randn(256, device=gpu, generator=gen) * 0.5).half()
+    ref = m.reference_step(token=7, pos=16, dequant=oracle_dequant)
+    _, logits = m.step(torch.tensor([7], device=gpu), torch.tensor([16], device=gpu), return_logits=True)
+    err = (logits[0].float() - ref).abs()
+    assert bool((err <= 1e-2 + 1e-3 * ref.abs()).all()), f"max err {err.max().item():.3g}"   # the matmul contract
+    for layer in m.layers:
+        layer["o"].bias = None
+    _, without = m.step(torch.tensor([7], device=gpu), torch.tensor([16], device=gpu), return_logits=True)
+    assert float((without.float() - logits.float()).abs().max()) > 0.1   # the bias reaches the logits
+
+
 def test_graph_replay_matches_eager(gpu):
     from metal_native.decoder import SyntheticDecoder
 
