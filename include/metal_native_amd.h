@@ -78,14 +78,18 @@ enum mq_epilogue {
  * itself when ldr == ldc (each element is read and then written by one
  * thread).  The kernels that split K across workgroups (the split-K GEMV,
  * the row-block GEMV when the activations exceed LDS, and the prefill GEMM
- * where its output tiles would leave most CUs idle) keep their partial sums
- * and counters in a library workspace per (device, stream), allocated by the
- * first call on that stream that needs it (so that call must not be inside
- * stream capture; under capture the prefill GEMM then keeps one workgroup per
- * tile instead).  Calls on one stream are ordered and share it.  When a
- * larger shape needs more, a new workspace replaces it for later calls; the
- * old one is kept (not freed) until the process ends, so graphs captured
- * earlier on that stream stay valid. */
+ * where its output tiles would leave CUs idle) keep their partial sums and
+ * counters in a library workspace per (device, stream), allocated by the first
+ * call on that stream that needs it (so that call must not be inside stream
+ * capture).  Under capture with a workspace too small, and where there is no
+ * memory for a larger one, the prefill GEMMs keep one workgroup per tile
+ * instead.  Calls on one stream are ordered and share it.  When a larger shape
+ * needs more, a new workspace replaces it for later calls; the old one is kept
+ * (not freed) until mq_release_workspaces or the process's end, so graphs
+ * captured earlier on that stream stay valid.  A stream's workspace is at most
+ * 64 MiB of partial sums for the prefill GEMMs and grows by doubling at least,
+ * so one stream holds at most about twice that; the option "workspace_mb"
+ * lowers the bound. */
 MQ_API int mq_dequant_matmul(const void* activations, int64_t lda, const void* weights_packed,
                              int64_t ldw_bytes, const void* scales, const void* zeros, void* out,
                              int64_t ldc, int64_t M, int64_t N, int64_t K, int32_t group_size,
@@ -255,6 +259,12 @@ MQ_API int mq_argmax_embed_f16(const void* logits, int64_t vocab, const void* em
 MQ_API int64_t mq_read_probe_sink_size(void);
 MQ_API int mq_read_probe(const void* p, int64_t bytes, void* sink, void* stream);
 
+/* Frees the workspaces of all streams, superseded ones too; later calls
+ * allocate anew.  Not while a call or a capture of the library is under way,
+ * and no graph captured before from a call that uses a workspace may be
+ * replayed afterwards (no reference counterpart). */
+MQ_API int mq_release_workspaces(void);
+
 /* Kernel-path override and layout knobs for tests and tuning (no reference
  * counterpart).  Keys: "force_path" (0 automatic, 2 the prefill GEMM family,
  * 3 generic, 6 split-K decode GEMV, 7 row-block decode GEMV, 12 register-
@@ -271,8 +281,10 @@ MQ_API int mq_read_probe(const void* p, int64_t bytes, void* sink, void* stream)
  * 0 automatic), both read when force_path is 13, "gemm_split" (1, the default: the 32x32x16 kernels split
  * K over several workgroups per output tile where its tiles would leave CUs
  * idle, summing the parts in a fixed order; 0: one workgroup per tile).  A forced path that cannot take the shape, or not
- * with these rows and parts, falls back to the automatic choice.  Returns MQ_INVALID_ARGUMENT for an unknown key or
- * value. */
+ * with these rows and parts, falls back to the automatic choice.  "workspace_mb": MiB that
+ * a stream's workspace may grow to, 0 (the default) no bound but the plans' own; a
+ * prefill GEMM that would need more runs without K parts, a split-K GEMV returns
+ * MQ_OUT_OF_MEMORY.  Returns MQ_INVALID_ARGUMENT for an unknown key or value. */
 MQ_API int mq_set_option(const char* key, int64_t value);
 
 /* Kernel the last successful mq_dequant_matmul / mq_vecmat_f16 /

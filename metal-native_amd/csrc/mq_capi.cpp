@@ -1,9 +1,11 @@
 // C-ABI entry points: argument validation (mirroring src/ops/matmul.mm:910-934),
 // kernel-path selection and launch.  The caller owns inputs and outputs; the
-// split-K GEMV's partial sums and counters live in a library workspace, one
-// per (device, stream), allocated and zeroed on first use and grown on demand.
+// counters and partial sums of the kernels that split K over workgroups live
+// in a library workspace, one per (device, stream), allocated on first use and
+// grown on demand.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdio>
 #include <cstring>
@@ -85,21 +87,28 @@ bool decode_ok(const mq::LinearArgs& a) {
   return mq::gemv_supported(a) && mq::gemv_plan(a, num_cus_current(), gemv_tuning()).ok;
 }
 
-// Split-K workspace, one per (device, stream): counters must start at zero and
-// every launch leaves them at zero, so one fill at allocation suffices.
-// Calls on one stream are ordered, so they may share it; mu is held from the
-// first to the last launch of a call that uses it, so that no other thread's
-// call on the stream comes between them (a many-row GEMM of several K parts
-// is two launches: the parts, and their sum).
+// Workspace of the kernels that split K over workgroups, one per (device,
+// stream): kWsCounters bytes of counters, which must start at zero and which
+// every launch leaves at zero, so one fill at allocation suffices; then
+// partial sums, which need no fill.  Calls on one stream are ordered, so they
+// may share it; mu is held from the first to the last launch of a call that
+// uses it, so that no other thread's call on the stream comes between them (a
+// many-row GEMM of several K parts is two launches: the parts, and their sum).
 struct Workspace {
   void* ptr = nullptr;
   size_t bytes = 0;
   std::mutex mu;
 };
+constexpr size_t kWsCounters = 65536;
 std::mutex g_ws_mu;
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
-std::vector<void*> g_ws_retired;   // superseded workspaces: kept until the process ends
+std::vector<void*> g_ws_retired;   // superseded workspaces: kept until mq_release_workspaces
+// workspace_mb: most bytes that a stream's workspace may grow to, 0 no bound
+// but the plans' own (mq::kMaxPartBytes)
+std::atomic<size_t> g_ws_limit{0};
 
+// hipErrorStreamCaptureUnsupported where the workspace would have to grow
+// under capture, hipErrorOutOfMemory where there is no memory for it.
 // `hold` locks the workspace where one is given out.
 hipError_t workspace_for(hipStream_t s, size_t need, void** out, std::unique_lock<std::mutex>& hold) {
   *out = nullptr;
@@ -114,18 +123,28 @@ hipError_t workspace_for(hipStream_t s, size_t need, void** out, std::unique_loc
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
       return hipErrorStreamCaptureUnsupported;  // first call on this stream must be outside capture
-    size_t nb = need < ((size_t)1 << 20) ? ((size_t)1 << 20) : need;
+    const size_t limit = g_ws_limit.load();
+    if (limit && need > limit) return hipErrorOutOfMemory;
     // A superseded buffer is kept, not freed: graphs captured earlier on
-    // this stream hold its address and may still be replayed.  Growth is
-    // geometric, so the retired buffers add up to less than the live one.
-    if (nb < 2 * w.bytes) nb = 2 * w.bytes;
+    // this stream hold its address and may still be replayed.  It doubles at
+    // least, up to what the largest plan needs, so the retired buffers add up
+    // to little more than the live one.
+    size_t nb = std::max({need, (size_t)1 << 20, std::min(2 * w.bytes, kWsCounters + mq::kMaxPartBytes)});
+    if (limit) nb = std::max(need, std::min(nb, limit));
     void* p = nullptr;
     e = hipMalloc(&p, nb);
-    if (e != hipSuccess) return e;
+    if (e == hipErrorOutOfMemory && nb > need) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, nb = need);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();   // not to be taken for that of the launch that follows
+      return e;
+    }
     // zeroed on the stream that uses it, so the first kernel on that stream
     // is ordered after the fill whatever the stream's flags (never inside a
     // capture: refused above)
-    e = hipMemsetAsync(p, 0, nb, s);
+    e = hipMemsetAsync(p, 0, std::min(nb, kWsCounters), s);
     if (e != hipSuccess) { (void)hipFree(p); return e; }
     if (w.ptr) g_ws_retired.push_back(w.ptr);
     w.ptr = p;
@@ -252,9 +271,9 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
   void* gn_ws = nullptr;
   if (path == PATH_GEMMN) {
     e = workspace_for(s, gn.ws_bytes, &gn_ws, hold);
-    if (e == hipErrorStreamCaptureUnsupported) {
-      // under capture with a workspace too small for this plan: the choice
-      // among the kernels that need none
+    if (e == hipErrorStreamCaptureUnsupported || e == hipErrorOutOfMemory) {
+      // a workspace too small for this plan under capture, or no memory for
+      // a larger one: the choice among the plans that need none
       path = choose_path(a, noalloc, false, &gn);
       e = hipSuccess;
     }
@@ -324,9 +343,10 @@ int run_linear(const mq::LinearArgs& a, hipStream_t s, bool noalloc = false) {
       void* ws = nullptr;
       size_t need = split ? mq::gemmw_ws_bytes(a, cus, true) : 0;
       hipError_t we = workspace_for(s, need, &ws, hold);
-      if (we == hipErrorStreamCaptureUnsupported) {
-        // under capture with a workspace too small for this shape: one
-        // workgroup per tile (no workspace) rather than an error
+      if (we == hipErrorStreamCaptureUnsupported || we == hipErrorOutOfMemory) {
+        // under capture with a workspace too small for this shape, or without
+        // memory for it: one workgroup per tile (no workspace) rather than an
+        // error
         split = false;
         need = 0;
         ws = nullptr;
@@ -771,6 +791,24 @@ MQ_API int mq_read_probe(const void* p, int64_t bytes, void* sink, void* stream)
   return MQ_SUCCESS;
 }
 
+MQ_API int mq_release_workspaces(void) {
+  std::lock_guard<std::mutex> lk(g_ws_mu);
+  hipError_t e = hipSuccess;
+  auto give_back = [&](void* p) {
+    const hipError_t fe = hipFree(p);   // waits for the work that uses it
+    if (fe != hipSuccess) e = fe;
+  };
+  for (void* p : g_ws_retired) give_back(p);
+  g_ws_retired.clear();
+  for (auto& [key, w] : g_ws) {
+    std::lock_guard<std::mutex> in_use(w.mu);
+    if (w.ptr) give_back(w.ptr);
+    w.ptr = nullptr;
+    w.bytes = 0;
+  }
+  return e == hipSuccess ? MQ_SUCCESS : hip_fail(e, "release_workspaces: freeing failed");
+}
+
 MQ_API int mq_set_option(const char* key, int64_t value) {
   if (!key) return fail(MQ_INVALID_ARGUMENT, "set_option: null key");
   if (std::strcmp(key, "force_path") == 0) {
@@ -800,6 +838,11 @@ MQ_API int mq_set_option(const char* key, int64_t value) {
   if (std::strcmp(key, "gemm_parts") == 0) {
     if (value < 0 || value > 64) return fail(MQ_INVALID_ARGUMENT, "set_option: gemm_parts must be 0..64");
     g_gemm_parts.store((int)value);
+    return MQ_SUCCESS;
+  }
+  if (std::strcmp(key, "workspace_mb") == 0) {
+    if (value < 0 || value > (int64_t)1 << 20) return fail(MQ_INVALID_ARGUMENT, "set_option: workspace_mb must be 0..1048576");
+    g_ws_limit.store((size_t)value << 20);
     return MQ_SUCCESS;
   }
   if (std::strcmp(key, "gemv_steps") == 0) {

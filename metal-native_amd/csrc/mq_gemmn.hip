@@ -630,7 +630,6 @@ bool gemmn_supported(const LinearArgs& a) {
 
 namespace {
 
-constexpr size_t kMaxPartBytes = (size_t)192 << 20;   // fp32 partial sums of one call
 // the start of the per-stream workspace holds the other kernels' counters,
 // which must stay zero
 constexpr size_t kCntBytesN = 65536;

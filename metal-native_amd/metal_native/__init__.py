@@ -13,7 +13,7 @@ from __future__ import annotations
 import types
 
 from .ops import (MetalNativeError, dequant_matmul, dequantize, last_path, matmul, quantize,
-                  set_option, swiglu, synchronize)
+                  release_workspaces, set_option, swiglu, synchronize)
 
 from . import nn, qformat  # noqa: E402  (layers, on-disk format and converters)
 from .qcache import QuantWeightCache  # noqa: E402
@@ -30,4 +30,4 @@ _C = types.SimpleNamespace(
 )
 
 __all__ = ["MetalNativeError", "dequant_matmul", "dequantize", "quantize", "matmul", "swiglu",
-           "fast", "synchronize", "set_option", "last_path", "_C", "nn", "qformat", "QuantWeightCache"]
+           "fast", "synchronize", "set_option", "last_path", "release_workspaces", "_C", "nn", "qformat", "QuantWeightCache"]

@@ -80,6 +80,7 @@ SIGNATURES = {
                                                   _c_void_p, _i32, _i32, _i32, _i64, ctypes.c_float, _c_void_p]),
     "mq_attention_parts_dequant_matmul": (_i32, [_c_void_p, _i32, _i32, _c_void_p, _i64, _c_void_p, _c_void_p,
                                                  _c_void_p, _i64, _i32, _i32, _c_void_p]),
+    "mq_release_workspaces": (_i32, []),
     "mq_set_option": (_i32, [ctypes.c_char_p, _i64]),
     "mq_last_path": (_i32, []),
     "mq_last_error": (ctypes.c_char_p, []),

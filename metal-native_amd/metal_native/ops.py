@@ -604,5 +604,12 @@ def set_option(key: str, value: int) -> None:
     _check(_L.mq_set_option(key.encode(), int(value)))
 
 
+def release_workspaces() -> None:
+    """Give back the device memory that the K-split kernels keep per stream
+    (``mq_release_workspaces``): not while calls are being made or captured,
+    and graphs captured before must not be replayed afterwards."""
+    _check(_L.mq_release_workspaces())
+
+
 def last_path() -> str:
     return _lib.PATH_NAMES.get(_L.mq_last_path(), "unknown")

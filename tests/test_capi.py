@@ -90,6 +90,16 @@ def test_set_option(lib):
     assert lib.mq_set_option(b"force_path", 0) == 0
 
 
+def test_set_option_of_the_many_row_gemm_and_workspace(lib):
+    for key, good, bad in ((b"gemm_rows", (64, 128, 256, 0), (32, -1)), (b"gemm_parts", (1, 64, 0), (65, -1)),
+                           (b"workspace_mb", (1, 1 << 20, 0), (-1, (1 << 20) + 1)), (b"force_path", (13, 0), (14,))):
+        for v in bad:
+            assert lib.mq_set_option(key, v) == 4 and key in lib.mq_last_error()
+        for v in good:
+            assert lib.mq_set_option(key, v) == 0
+    assert lib.mq_release_workspaces() == 0   # nothing held
+
+
 def test_python_surface_mirrors_reference():
     import metal_native as mn
 

@@ -250,6 +250,50 @@ def test_capture_and_shared_workspace(mn, gpu):
             check(got.cpu().numpy(), vref, what="split-K GEMV between replays")
 
 
+@pytest.mark.parametrize("M,K,N,epi,parts_path", [(300, 8192, 2048, None, "gemmn"), (37, 18944, 3584, "residual", "gemmn"),
+                                                  (64, 3104, 256, "bias", "gemmw_split")])
+def test_no_memory_for_a_workspace(mn, gpu, M, K, N, epi, parts_path):
+    """Where a stream's workspace cannot grow, a plan without K parts runs;
+    once it can, the K parts again."""
+    x, wp, s, z, g, acc = problem(M, K, N, 32, "int4", seed=N)
+    kw, b, r = epilogue_args(epi, M, N, gpu)
+    args = dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, "int4"
+    mn.release_workspaces()
+    # (bounds below each plan's partial sums; 1 MiB is the smallest)
+    stream = torch.cuda.Stream(gpu)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        mn.set_option("gemm_split", 0)
+        want = mn.dequant_matmul(*args, **kw)
+        path = mn.last_path()
+        mn.set_option("gemm_split", 1)
+        mn.set_option("workspace_mb", 1)
+        try:
+            got = mn.dequant_matmul(*args, **kw)
+            without = mn.last_path()
+        finally:
+            mn.set_option("workspace_mb", 0)
+        again = mn.dequant_matmul(*args, **kw)
+        assert mn.last_path() == parts_path
+    torch.cuda.synchronize()
+    if parts_path == "gemmn":   # (the third plan's partial sums fit in 1 MiB)
+        assert without == path and torch.equal(got, want)
+    for y in (got, again):
+        check(y.cpu().numpy(), acc, epi, b, r, path)
+
+
+def test_release_workspaces(mn, gpu):
+    M, K, N, g = 777, 18944, 3584, 128   # 43 MiB of partial sums
+    args = tuple(dev(a, gpu) for a in O.make_int4_problem(M, K, N, g, seed=2)) + (g, "int4")
+    want = mn.dequant_matmul(*args)
+    assert mn.last_path() == "gemmn"
+    torch.cuda.synchronize()
+    held = torch.cuda.mem_get_info(gpu)[0]
+    mn.release_workspaces()
+    assert torch.cuda.mem_get_info(gpu)[0] - held >= 40 << 20
+    assert torch.equal(mn.dequant_matmul(*args), want)
+
+
 def test_threads_on_one_stream(mn, gpu):
     """Calls of several K parts (two launches that share the stream's
     workspace) from threads on one stream, among calls of the split-K GEMV on
