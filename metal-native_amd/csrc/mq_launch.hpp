@@ -102,7 +102,7 @@ struct RowsPlan {
   int KP, nblk, KStot;
   uint32_t off_sz, off_scr, off_slot, off_wft;
   size_t lds_bytes, ws_bytes;
-  bool ok;
+  bool ok, fast;   // fast: int4 by the 13-op dequant where the scales allow it
 };
 RowsPlan rows_plan(const LinearArgs& a, int num_cus, bool allow_split = true);
 hipError_t rows_launch(const LinearArgs& a, const RowsPlan& p, void* ws, hipStream_t s);

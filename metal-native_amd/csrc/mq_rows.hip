@@ -61,6 +61,17 @@ constexpr int ring_depth() { return FMT == FMT_INT4 ? 3 : 4; }
 // in total, 3-4 % slower at 34 MB and more)
 constexpr int kNWBig = 12, kNWSmall = 8;
 constexpr int64_t kSmallBytes = 64 * 1024;
+// The 13-op int4 dequant: in the twelve-wave builds (more than kSmallBytes), up
+// to M = 8; for M = 9..16, which take twelve waves at any size, where the
+// workgroup streams more than kFastBytesMh2.  With its range test and a second
+// loop for other scales the start of a launch is 0.1-0.3 us longer, and the
+// stream of a large layer shorter by more than that.  With it / without, graph
+// timing, 256 workgroups: M = 1 K = 4096, N = 14336 (112 KiB of weights each)
+// 9.66 / 10.06 us, K = 3584, N = 37888 16.8 / 17.5; M = 2 K = 3072, N = 12288
+// (72 KiB) 8.33 / 8.55; eight waves, 7B QKV 8.0 / 7.7, o_proj 5.80 / 5.74.  M
+// = 13: K = N = 1024 8.34 / 8.11, K = 4096, N = 12288 (96 KiB) 13.89 / 13.73,
+// N = 14336 (112 KiB) 15.03 / 15.15, K = 3584, N = 37888 24.4 / 25.1.
+constexpr int64_t kFastBytesMh2 = 104 * 1024;
 static_assert(kNWBig % 4 == 0 && kNWSmall % 4 == 0, "the slot sums read the first-tile table in groups of four");
 constexpr int kPre = 2;      // ring slots issued before the staging data is waited for
 constexpr int kXB = 8;           // activation pieces per thread per staging batch
@@ -94,8 +105,9 @@ struct RowsKArgs {
 };
 
 // PRE: 0 the activations as they are, 1 the fused residual add + RMSNorm, 2 the
-// fused combine of attention partials (M = 1 both)
-template <int FMT, int EPI, int RPW, int PRE, int NW, int MH>
+// fused combine of attention partials (M = 1 both).  FASTDQ: int4 by the 13-op
+// dequant where all staged scales are in its range (RowsPlan::fast).
+template <int FMT, int EPI, int RPW, int PRE, int NW, int MH, bool FASTDQ>
 __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   constexpr int S = 16 / RPW;
   constexpr int KPL = FmtTraits<FMT>::KPL;       // k per 16-byte piece
@@ -105,12 +117,6 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   constexpr int BPK2 = (FMT == FMT_INT4) ? 1 : (FMT == FMT_INT8 ? 2 : 4);  // 2 x bytes per k
   extern __shared__ __align__(16) unsigned char smem[];
 
-  // The 13-op dequant, in the twelve-wave builds: with its range test and a
-  // second loop for other scales the start of a launch is ~0.3 us longer, and
-  // the stream of 34 MB and more shorter by more than that (7B gate/up 17.9 ->
-  // 17.4 us, lm_head 57.2 -> 54.2, down 11.8 -> 11.5; QKV and o_proj, eight
-  // waves, 7.7 -> 8.0 and 5.74 -> 5.80 us).
-  constexpr bool FASTDQ = FMT == FMT_INT4 && NW == kNWBig;
   constexpr int NT = 64 * NW;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -433,9 +439,9 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   }
 #pragma unroll
   for (int d = kPre; d < kD; ++d) raw[d] = wload();
-  {
-    const int bad = FASTDQ && __builtin_amdgcn_ballot_w64(fast_scale_bad(smax)) != 0 ? INT_MIN : 0;
-    if (lane == 0) wft[w] = (u0 / KS) | bad;   // the tiles are read by the slot sums after the final barrier
+  if constexpr (FASTDQ) {
+    const int bad = __builtin_amdgcn_ballot_w64(fast_scale_bad(smax)) != 0 ? INT_MIN : 0;
+    if (lane == 0) wft[w] = (u0 / KS) | bad;
   }
   // LDS barrier that leaves the weight loads in flight
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -452,6 +458,7 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
 
   int ct = u0 / KS, cj = u0 - ct * KS;   // consume cursor (tile, step)
   const int ft = ct;                      // first tile of this wave
+  if (!FASTDQ && lane == 0) wft[w] = ft;  // read by the slot sums after the final barrier
   // scale entry of the lane's row and group: the step advances it by a
   // uniform KSTEP / g groups.  In a row's last step, lanes whose k lies past
   // K would reach the next row's entries: they keep their own row's last
@@ -682,9 +689,9 @@ __global__ __launch_bounds__(64 * NW) void rows_kernel(RowsKArgs p) {
   }
 }
 
-template <int FMT, int EPI, int RPW, int PRE, int NW, int MH>
+template <int FMT, int EPI, int RPW, int PRE, int NW, int MH, bool FASTDQ>
 hipError_t launch5(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
-  auto fn = rows_kernel<FMT, EPI, RPW, PRE, NW, MH>;
+  auto fn = rows_kernel<FMT, EPI, RPW, PRE, NW, MH, FASTDQ>;
   hipError_t e = allow_dynamic_lds((const void*)fn, (int)kLds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(pl.nwg), dim3(64 * NW), pl.lds_bytes, s, k);
@@ -695,7 +702,10 @@ template <int FMT, int EPI, int RPW, int PRE>
 hipError_t launch4(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
   if constexpr (RPW == 8 && !PRE && FMT != FMT_F16) {
     if (pl.mh == 2) {   // M = 9..16 on 8-row tiles: twelve waves (the activations are large)
-      if (pl.nw == kNWBig) return launch5<FMT, EPI, RPW, PRE, kNWBig, 2>(k, pl, s);
+      if constexpr (FMT == FMT_INT4) {
+        if (pl.fast) return launch5<FMT, EPI, RPW, PRE, kNWBig, 2, true>(k, pl, s);
+      }
+      if (pl.nw == kNWBig) return launch5<FMT, EPI, RPW, PRE, kNWBig, 2, false>(k, pl, s);
       return hipErrorInvalidValue;
     }
   }
@@ -703,9 +713,9 @@ hipError_t launch4(const RowsKArgs& k, const RowsPlan& pl, hipStream_t s) {
   // (int8 with the pre-norm always takes twelve waves: its eight-wave build
   // spills registers)
   if constexpr (!(FMT == FMT_INT8 && PRE)) {
-    if (pl.nw == kNWSmall) return launch5<FMT, EPI, RPW, PRE, kNWSmall, 1>(k, pl, s);
+    if (pl.nw == kNWSmall) return launch5<FMT, EPI, RPW, PRE, kNWSmall, 1, false>(k, pl, s);
   }
-  if (pl.nw == kNWBig) return launch5<FMT, EPI, RPW, PRE, kNWBig, 1>(k, pl, s);
+  if (pl.nw == kNWBig) return launch5<FMT, EPI, RPW, PRE, kNWBig, 1, FMT == FMT_INT4>(k, pl, s);
   return hipErrorInvalidValue;
 }
 
@@ -815,6 +825,7 @@ RowsPlan rows_plan_k(const LinearArgs& a, int num_cus, int KP) {
   const int U = TW * KS;
   const int64_t wbytes = (int64_t)(a.epi == EPI_SWIGLU ? 2 * R : R) * a.ldw / KP;   // weight bytes per workgroup
   const int nw = mh == 2 || wbytes > kSmallBytes || (a.prenorm && a.fmt == FMT_INT8) ? kNWBig : kNWSmall;
+  p.fast = a.fmt == FMT_INT4 && nw == kNWBig && (mh == 1 || wbytes > kFastBytesMh2);
   const int per = (U + nw - 1) / nw;
   const int maxT = per / KS + 2;
   if ((int64_t)(a.epi == EPI_SWIGLU ? a.F + R : R) * a.ldw >= lim) return p;
