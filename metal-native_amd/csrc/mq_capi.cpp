@@ -177,11 +177,14 @@ bool gemm16_auto(const mq::LinearArgs& a) {
 // The many-row GEMM (mq_gemmn.hip), automatically: where its launch-time
 // model is at least 7 % below that of the kernel the shape would take
 // otherwise, and that one is 19 us or more (below, it was the slower one on
-// every shape).  On 208 shapes with M = 32..4096 and 148 with M = 17..512 the
-// choice is the faster kernel, or within 6 % of it, on all but 12: e.g. M =
-// 4096, K = 3584, N = 37888 int4 SwiGLU 1.05 ms against 2.51; M = 777, K =
-// 18944, N = 3584 134 us against 275; M = 37 there 28 against 33; M = 512,
-// K = 3072, N = 5120 stays with the 16x16x32 GEMM (23 against 35 us).
+// most shapes).  On 1000 drawn shapes that the models were not fitted to (M =
+// 17..4096, K = 512..18944, N = 512..37888) it takes 483: it is the slower
+// kernel by more than 5 % on 4 of them (11 % at most: M = 31, K = 6176, N =
+// 17500 int8, 36.4 against 32.8 us) and 2.4 times as fast on the mean; of the
+// 517 others it would be more than 5 % faster on 64.  M = 4096, K = 3584, N =
+// 37888 int4 SwiGLU 1.05 ms against 2.51; M = 777, K = 18944, N = 3584 134 us
+// against 275; M = 37 there 27 against 33; M = 512, K = 3072, N = 5120 stays
+// with the 16x16x32 GEMM (23 against 35 us).
 mq::GemmnPlan gemmn_auto(const mq::LinearArgs& a, bool allow_split) {
   const int cus = num_cus_current();
   allow_split = allow_split && g_gemm_split.load() != 0;

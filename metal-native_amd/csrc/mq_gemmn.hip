@@ -635,34 +635,45 @@ namespace {
 constexpr size_t kCntBytesN = 65536;
 
 // Launch-time model (microseconds), fitted to 774 (256-row tiles) and 1056
-// (128-row tiles) measured launches: M = 32..4096, K = 896..18944, N =
-// 896..37888, int4 and int8, 1-16 K parts; 5 % rms, at most 24 % off.
+// (128-row tiles) measured launches (M = 32..4096, K = 896..18944, N =
+// 896..37888, int4 and int8, 1-16 K parts, 5 % rms) and refitted with 1700
+// launches of drawn shapes (K = 512..18944, N = 512..37888, all group sizes and
+// epilogues), where it is 8 % off with K parts; without them 128- and 256-row
+// tiles take a quarter longer than it says, on shapes where the other kernels
+// are further off still.
 //  * 256 rows: one workgroup per CU.  A K-tile takes 1.22 us, and up to 1.70
 //    us when all CUs run (the clock drops under the load).
 //  * 128 rows: two workgroups fit a CU; a K-tile takes 0.77-1.05 us alone,
 //    2.02 us in each of two.
-//  * 64 rows: two workgroups fit a CU; a K-tile takes 0.71 us alone, 1.05 us in
-//    each of two (1414 launches, M = 17..512, 7 % rms).
-//  * K parts: their sums are written and read once, 0.145 us per MB.
-double estimate(int mb, int64_t wgs, int ktp, double part_mb, double weight_mb, int cus) {
-  const double split = part_mb > 0.0 ? 1.0 : 0.0;
+//  * 64 rows: two workgroups fit a CU; a K-tile takes 0.70 us alone, 1.07 us in
+//    each of two (int8 0.10 and 0.30 more), and the bytes of scales, outputs
+//    and residual count (2536 launches, M = 17..512, 8 % rms).
+//  * K parts: their sums are written and read once, 0.14-0.22 us per MB, and a
+//    thread adds all parts of its 8 columns, 0.1 us a part, or 0.5 with SwiGLU
+//    (half the threads with twice the loads; where they are few, nothing hides
+//    the loads' latency: M = 107, K = 4864, N = 896 in 19 parts takes 22 us, 14
+//    without this term).
+double estimate(const LinearArgs& a, int mb, int64_t wgs, int KP, int ktp, double part_mb, int cus) {
+  const bool swi = a.epi == EPI_SWIGLU, i8 = a.fmt == FMT_INT8;
+  const double split = KP > 1 ? 1.0 : 0.0, sum = split * (swi ? 0.47 : 0.10) * KP;
   if (mb == 8) {
     const double rounds = (double)wgs / cus;
     const double whole = std::ceil(rounds);
     const double tk = 1.22 + 0.48 * std::max(0.0, std::min(1.0, rounds) - 0.5) * 2.0;
-    return 11.3 + (whole <= 3 ? whole : rounds + 0.5) * (1.97 + ktp * tk) + split * 0.29 + 0.143 * part_mb;
+    return 11.3 + (whole <= 3 ? whole : rounds + 0.5) * (1.97 + ktp * tk) + split * 0.29 + 0.143 * part_mb + sum;
   }
   const int64_t slots = 2 * (int64_t)cus;
   const int64_t full = wgs / slots, rem = wgs - full * slots;
   if (mb == 2) {
-    double t = (full + (rem > cus ? 1 : 0)) * (ktp * 1.053 - 1.57);
-    if (rem > 0 && rem <= cus) t += ktp * 0.709 * (1.0 + 0.009 * (double)rem / cus) - 1.57;
-    return 6.72 + std::max(0.0, t) + 0.09 * weight_mb + split * 2.46 + 0.231 * part_mb;
+    const double scale_mb = 4e-6 * a.N * a.G, out_mb = 2e-6 * a.M * (swi ? a.N / 2 : a.N);
+    return 5.12 + (full + (rem > cus ? 1 : 0)) * ktp * (i8 ? 1.372 : 1.068) +
+           (rem > 0 && rem <= cus ? ktp * (i8 ? 0.796 : 0.696) : 0.0) + 0.756 * scale_mb + 0.729 * out_mb +
+           (a.epi == EPI_RESIDUAL ? 1.05 * out_mb : 0.0) + split * (1.51 + (swi ? 0.509 : 0.133) * KP) + 0.222 * part_mb;
   }
   double t = 8.05 + full * (1.55 + ktp * 2.02);
   if (rem > cus) t += 1.55 + ktp * (0.77 + 1.25 * (0.6 + 0.4 * (double)(rem - cus) / cus));
   else if (rem > 0) t += 1.55 + ktp * 0.77 * (1.0 + 0.36 * (double)rem / cus);
-  return t + split * 1.06 + 0.148 * part_mb;
+  return t + split * (swi ? -0.62 : 0.45) + 0.19 * part_mb + sum;
 }
 
 }  // namespace
@@ -674,7 +685,6 @@ GemmnPlan gemmn_plan(const LinearArgs& a, int cus, bool allow_split, int mb, int
   const int F = swi ? a.F : a.N;
   const int KT = (a.K + 63) / 64;
   const int64_t ld = (int64_t)((F + 7) & ~7) * (swi ? 2 : 1);
-  const double wmb = (double)a.N * a.K * (a.fmt == FMT_INT4 ? 0.5e-6 : 1e-6);
   for (int m = 2; m <= 8; m *= 2) {
     if (mb ? m != mb : m == 2 && a.M > 320) continue;   // (64 rows: not the fastest beyond, and not modelled)
     const int64_t tiles = (int64_t)((a.M + 32 * m - 1) / (32 * m)) * ((F + (swi ? 127 : 255)) / (swi ? 128 : 256));
@@ -686,7 +696,7 @@ GemmnPlan gemmn_plan(const LinearArgs& a, int cus, bool allow_split, int mb, int
       if (tiles * KP > 0x7fffffff / 256) continue;
       const size_t part = KP > 1 ? (size_t)KP * a.M * ld * 4 : 0;
       if (part > kMaxPartBytes) continue;
-      const double t = estimate(m, tiles * KP, ktp, 2.0 * (double)part / 1e6, wmb, cus);
+      const double t = estimate(a, m, tiles * KP, KP, ktp, 2.0 * (double)part / 1e6, cus);
       if (!best.ok || t < best.us) best = GemmnPlan{m, KP, ktp, part ? kCntBytesN + part : 0, t, true};
     }
   }

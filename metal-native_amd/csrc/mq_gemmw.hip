@@ -552,10 +552,6 @@ bool sz_table_fits(const LinearArgs& a, int BN) {
   return (int64_t)(a.epi == EPI_SWIGLU ? 2 * BN : BN) * a.G <= SZT;
 }
 
-// Time model of one tile (microseconds at ~2.1 GHz): MFMA issue, dequant
-// VALU, texture-unit requests and the tile's weight bytes at its share of
-// ~6 TB/s; the launch takes ceil(tiles / CUs) tile times (one workgroup per
-// CU).
 // Launch time (us) of MB x NB tiles with KP K parts each: fitted to 290
 // measured launches (int4, M = 17..128, K = 2048..18944): per-wave K-tiles
 // times the tile's MFMA, dequant and activation work, rounds of workgroups
@@ -570,6 +566,10 @@ double launch_us(int K, int MB, int NB, int64_t tiles, int KP, int cus) {
          11.39 * rounds;
 }
 
+// One part per tile: a time model of one tile (microseconds at ~2.1 GHz) of
+// MFMA issue, dequant VALU, texture-unit requests and the tile's weight bytes
+// at its share of ~6 TB/s; the launch takes ceil(tiles / CUs) tile times (one
+// workgroup per CU).  K parts: by launch_us.
 WPlan plan(const LinearArgs& a, int cus, bool allow_split) {
   WPlan best{};
   best.ok = false;
@@ -706,22 +706,27 @@ bool gemmw_supported(const LinearArgs& a, int cus) {
 
 size_t gemmw_ws_bytes(const LinearArgs& a, int cus, bool allow_split) { return plan(a, cus, allow_split).ws_bytes; }
 
-// Per format, fitted to 117 (int4) and 62 (int8) measured launches up to M =
-// 4096 (10 % and 7 % rms; launch_us, which only ranks this kernel's own
-// tilings, is 14 % and 10 % off there): a round of workgroups costs a fixed
-// time and its per-wave K-tiles times the work of an MB x NB tile.
+// Per format and tile shape, fitted to 1217 (int4) and 661 (int8) measured
+// launches of drawn shapes (M = 17..4096, K = 544..18944, N = 512..37888; 12 %
+// and 13 % rms; launch_us, which only ranks this kernel's own tilings, is
+// further off there): a round of workgroups costs a fixed time and its
+// per-wave K-tiles times the tile's own, a little more when the rounds are
+// full; a residual is read element by element.
 double gemmw_estimate(const LinearArgs& a, int cus, bool allow_split) {
   const WPlan p = plan(a, cus, allow_split);
   if (!p.ok) return 0.0;
   const bool i4 = a.fmt == FMT_INT4;
-  const double c0 = i4 ? -2.05 : 1.03, c1 = i4 ? 7.63 : 6.93, k0 = i4 ? 19.25 : 18.65, kmn = i4 ? 4.94 : 4.78;
-  const double kn = i4 ? -9.43 : -9.11, km = i4 ? -9.66 : -9.42, load = i4 ? 0.006 : 0.054;
-  const double s0 = i4 ? 1.43 : -1.70, s1 = i4 ? 0.207 : 0.258;
+  // us per K-tile of a wave; the shapes that plan() takes: MB x NB = 1 x 2, 2 x 2, 2 x 3, 2 x 4, 2 x 6, 4 x 2, 4 x 3
+  static const double tile4[7] = {0.389, 0.662, 1.140, 1.818, 2.602, 1.225, 2.212};
+  static const double tile8[7] = {0.499, 0.623, 1.217, 1.553, 2.880, 1.281, 1.872};
+  const int shape = p.MB == 1 ? 0 : p.MB == 2 ? (p.NB == 6 ? 4 : p.NB - 1) : p.NB + 3;
   const double per = std::ceil(a.K / 64.0) / p.KP / 4.0, mn = (double)p.MB * p.NB;
-  const double r = (double)((int64_t)p.nbm * p.nbn * p.KP) / cus;
-  const double rounds = std::ceil(r) <= 3.0 ? std::ceil(r) : r + 0.5;
-  const double tile = k0 + kmn * mn + kn * p.NB + km * p.MB + load * mn * std::min(1.0, std::max(0.0, r - 0.5));
-  return c0 + rounds * (c1 + per * tile) + (p.KP > 1 ? s0 + s1 * p.KP * mn : 0.0);
+  const double r = (double)((int64_t)p.nbm * p.nbn * p.KP) / cus, r1 = r / p.KP;
+  auto rounds = [](double x) { return std::ceil(x) <= 3.0 ? std::ceil(x) : x + 0.5; };
+  const double tile = (i4 ? tile4 : tile8)[shape] + (i4 ? 0.0173 : 0.0237) * mn * std::min(1.0, std::max(0.0, r - 0.5));
+  return rounds(r) * ((i4 ? 6.84 : 7.25) + per * tile) +
+         (p.KP > 1 ? (i4 ? 2.18 : 2.44) + (i4 ? 0.175 : 0.153) * p.KP * mn : 0.0) +
+         (a.epi == EPI_RESIDUAL ? (i4 ? 0.623 : 0.675) * mn * rounds(r1) : 0.0);
 }
 
 hipError_t gemmw_launch(const LinearArgs& a, int cus, void* ws, hipStream_t s, bool allow_split) {

@@ -218,6 +218,26 @@ def test_routing(mn, gpu, M, K, N, g, qt, epi, want):
     check(y.cpu().numpy(), acc, epi, b, r, want)
 
 
+@pytest.mark.parametrize("M,K,N,g,qt,epi", [   # us: the kernel it is left to / this one
+    (1941, 1120, 1298, 32, "int8", None),      # 21.0 / 28.1
+    (117, 3424, 23562, 3424, "int8", None),    # 44.2 / 53.7
+    (19, 2144, 25754, 32, "int4", "swiglu"),   # 26.6 / 35.1
+    (107, 4864, 896, 128, "int4", "swiglu"),   # 18.9 / 22.2: many K parts for few threads to add
+    (93, 2304, 21770, 64, "int4", None),       # 27.6 / 31.9
+    (452, 2336, 4572, 32, "int4", None),       # 28.2 / 32.1
+])
+def test_routing_leaves_the_faster_kernel(mn, gpu, M, K, N, g, qt, epi):
+    x = torch.randn((M, K), device=gpu).half()
+    w = torch.randint(0, 256, (N, K // 2 if qt == "int4" else K), dtype=torch.uint8, device=gpu)
+    s = torch.full((N, K // g), 0.01, dtype=torch.float16, device=gpu)
+    args = (x, w if qt == "int4" else w.view(torch.int8), s, s, g, qt)
+    got = mn.dequant_matmul(*args, epilogue=epi)
+    assert mn.last_path() in ("gemmw", "gemmw_split", "gemm16"), mn.last_path()
+    if epi is None:
+        ref = x.float() @ mn.dequantize(*args[1:]).float().t().contiguous()
+        assert bool(((got.float() - ref).abs() <= TOL_ABS + TOL_REL * ref.abs()).all())
+
+
 def test_capture_and_shared_workspace(mn, gpu):
     """K parts under capture: with the stream's workspace in place the graph
     replays them; on a fresh stream a kernel without one runs.  The split-K
@@ -228,6 +248,13 @@ def test_capture_and_shared_workspace(mn, gpu):
     v = O.make_int4_problem(1, 896, 4864, 64, seed=8)
     vref = O.matmul_f32acc(v[0], O.dequant_int4(v[1], v[2], v[3], 896, 64))
     vargs = tuple(dev(a, gpu) for a in v) + (64, "int4")
+    eager = {True: mn.dequant_matmul(*args)}
+    assert mn.last_path() == "gemmn"
+    mn.set_option("gemm_split", 0)
+    eager[False] = mn.dequant_matmul(*args)
+    path = {True: "gemmn", False: mn.last_path()}
+    mn.set_option("gemm_split", 1)
+    assert not torch.equal(eager[True], eager[False])   # the parts show in the rounding
     for warm in (True, False):
         stream = torch.cuda.Stream(gpu)
         stream.wait_stream(torch.cuda.current_stream(gpu))
@@ -239,11 +266,14 @@ def test_capture_and_shared_workspace(mn, gpu):
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=stream):
             y = mn.dequant_matmul(*args)
+            captured = mn.last_path()
+        assert captured == path[warm]
         for _ in range(3):
             y.zero_()
             graph.replay()
             torch.cuda.synchronize()
             check(y.cpu().numpy(), acc, what=f"replay warm={warm}")
+            assert torch.equal(y, eager[warm])
             with torch.cuda.stream(stream):
                 got = mn.dequant_matmul(*vargs)
             torch.cuda.synchronize()
