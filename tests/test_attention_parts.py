@@ -154,6 +154,25 @@ def test_error_against_float64_no_larger(gpu):
     assert worst[1] <= 2.0**-10 and worst[1] <= 1.01 * worst[0]
 
 
+def test_fused_branch_runs_where_supported(gpu, monkeypatch):
+    """The two-call form is not behind a supported shape's output."""
+    from metal_native import ops
+
+    H, KVH, D, L = 8, 2, 128, 576
+    cos, sin, kc, vc, qkv, o = _case(gpu, H, KVH, D, L, 640, seed=6)
+    args = (qkv, cos, sin, torch.tensor([500], device=gpu), kc, vc, H, KVH, D, 1.0 / math.sqrt(D))
+    want = ops.dequant_matmul(ops.attention_decode_rope(*args), *o.operands())
+
+    def refuse(*a, **k):
+        raise AssertionError("the general branch ran")
+
+    monkeypatch.setattr(ops, "attention_decode_rope", refuse)
+    got = ops.attention_decode_rope_linear(*args, *o.operands())
+    assert float((got - want).double().norm() / want.double().norm()) < 1e-3   # fp16 roundings, 2^-11 each
+    with pytest.raises(AssertionError, match="general branch"):
+        ops.attention_decode_rope_linear(*args, *o.operands(), bias=want[0])
+
+
 def test_graph_replays(gpu):
     from metal_native import ops
 

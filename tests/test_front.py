@@ -98,6 +98,59 @@ def test_front_equals_the_general_path(mn, gpu, quant, g, epilogue):
 
 
 @pytest.mark.gpu
+def test_front_takes_or_declines(gpu):
+    """Which calls the front takes (an output) and which it leaves to the
+    general path (None)."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from metal_native import _mq_torch
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, w, s, z = problem(gpu)
+    stream = torch.cuda.current_stream(gpu).cuda_stream
+    a, b = torch.randn((2, 512), device=gpu).half(), torch.randn((300, 512), device=gpu).half()
+
+    def linear(x=x, w=w, s=s, z=z, g=64, int4=True, epi=0, bias=None, resid=None):
+        return _mq_torch.dequant_matmul(x, w, s, z, g, int4, epi, bias, resid, stream)
+
+    def vecmat(a=a, b=b, tb=True):
+        return _mq_torch.vecmat(a, b, tb, stream)
+
+    strided = lambda t: torch.stack((t, t), -1)[..., 0]
+    row = lambda t: torch.nn.Parameter(t, requires_grad=False)
+    resid = torch.randn((3, 384), device=gpu).half()
+    for take in (lambda: linear(), lambda: linear(wider(x), wider(w)), lambda: linear(row(x), row(w), row(s), row(z)),
+                 lambda: linear(x.clone().requires_grad_()), lambda: linear(epi=5),
+                 lambda: linear(epi=1, bias=resid[0].contiguous()), lambda: linear(epi=4, resid=wider(resid)),
+                 lambda: vecmat(), lambda: vecmat(wider(a), wider(b)), lambda: vecmat(a, b.t().contiguous(), False),
+                 lambda: vecmat(a.float(), b.float())):
+        assert type(take()) is torch.Tensor
+    for decline in (lambda: linear(x.as_subclass(Marked)), lambda: linear(strided(x)), lambda: linear(w=strided(w)),
+                    lambda: linear(s=strided(s)), lambda: linear(s=wider(s)), lambda: linear(x[:1].expand(3, 512)),
+                    lambda: linear(x[0]), lambda: linear(x.float()), lambda: linear(x.cpu()), lambda: linear(s=s[1:]),
+                    lambda: linear(g=48), lambda: linear(int4=False), lambda: linear(epi=1), lambda: linear(bias=s[0]),
+                    lambda: linear(epi=7), lambda: linear(epi=4, resid=strided(resid)), lambda: linear(x[:0]),
+                    lambda: vecmat(a[0]), lambda: vecmat(strided(a)), lambda: vecmat(a.as_subclass(Marked)),
+                    lambda: vecmat(a, b.float()), lambda: vecmat(a[:, :200], b[:, :200]), lambda: vecmat(a, b[:200]),
+                    lambda: vecmat(a.repeat(5, 1)), lambda: vecmat(a, b.cpu())):
+        assert decline() is None
+    for mode in (Function(), Dispatch()):
+        with mode:
+            assert linear() is None and vecmat() is None
+    seen = []
+    torch.func.vmap(lambda v: (seen.append((linear(v), vecmat(a, v))), v)[1])(torch.stack((x, x)))
+    assert seen == [(None, None)]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("transpose_b", [True, False])
 @pytest.mark.parametrize("M", [1, 8])
