@@ -174,16 +174,17 @@ bool gemm16_auto(const mq::LinearArgs& a) {
   return 4 * (int64_t)mq::gemm16_workgroups(a) >= 3 * (int64_t)num_cus_current() && 4 * (int64_t)a.M >= 3 * mpad;
 }
 
-// The many-row GEMM (mq_gemmn.hip), automatically: where its launch-time
-// model is at least 7 % below that of the kernel the shape would take
-// otherwise, and that one is 19 us or more (below, it was the slower one on
-// most shapes).  On 1000 drawn shapes that the models were not fitted to (M =
-// 17..4096, K = 512..18944, N = 512..37888) it takes 483: it is the slower
-// kernel by more than 5 % on 4 of them (11 % at most: M = 31, K = 6176, N =
-// 17500 int8, 36.4 against 32.8 us) and 2.4 times as fast on the mean; of the
-// 517 others it would be more than 5 % faster on 64.  M = 4096, K = 3584, N =
-// 37888 int4 SwiGLU 1.05 ms against 2.51; M = 777, K = 18944, N = 3584 134 us
-// against 275; M = 37 there 27 against 33; M = 512, K = 3072, N = 5120 stays
+// The many-row GEMM (mq_gemmn.hip), automatically: by launch-time models,
+// against the kernel the shape would take otherwise, where that one is 19 us
+// or more (below, this one is the slower on 401 of 486 drawn shapes).  The
+// margins are where the two cross on 6000 drawn shapes (M = 17..4096, K =
+// 512..18944, N = 512..37888): 2 % above the estimate of the 16x16x32 GEMM and
+// of the 32x32x16 GEMM with K parts, 5 % below that of the latter without.
+// There it takes 2483, 2.0 times as fast (geometric mean), and is the slower
+// kernel by more than 5 % on 35 of them, by 31 % at most (M = 22, K = 6336, N =
+// 18280: two workgroups per CU take longer than modelled).  M = 4096, K = 3584,
+// N = 37888 int4 SwiGLU 1.05 ms against 2.51; M = 777, K = 18944, N = 3584 134
+// us against 275; M = 37 there 27 against 33; M = 512, K = 3072, N = 5120 stays
 // with the 16x16x32 GEMM (23 against 35 us).
 mq::GemmnPlan gemmn_auto(const mq::LinearArgs& a, bool allow_split) {
   const int cus = num_cus_current();
@@ -191,15 +192,19 @@ mq::GemmnPlan gemmn_auto(const mq::LinearArgs& a, bool allow_split) {
   mq::GemmnPlan none{};
   if (a.M <= 16 || g_gemm_impl.load() != 0 || !mq::gemmn_supported(a)) return none;
   double other = 1e30;   // the 16x16x32 kernel's fallback: always slower
+  double margin = 0.95;
   if (gemm16_auto(a)) {
     if (mq::gemm16_rows_per_tile(a) != 128) return none;   // 64-row SwiGLU tiles: made for M <= 64
     other = mq::gemm16_estimate(a, cus);
+    margin = 1.02;
   } else if (mq::gemmw_supported(a, cus)) {
-    other = mq::gemmw_estimate(a, cus, allow_split);
+    bool parts = false;
+    other = mq::gemmw_estimate(a, cus, allow_split, &parts);
+    if (parts) margin = 1.02;
   }
   if (other < 19.0) return none;
   const mq::GemmnPlan p = mq::gemmn_plan(a, cus, allow_split);
-  return p.ok && p.us < 0.93 * other ? p : none;
+  return p.ok && p.us < margin * other ? p : none;
 }
 
 // Short weight rows over many of them, M <= 4: the split-K GEMV, whose

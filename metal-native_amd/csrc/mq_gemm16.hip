@@ -675,14 +675,19 @@ int gemm16_workgroups(const LinearArgs& a) {
   return ((a.M + 16 * sh.mbk - 1) / (16 * sh.mbk)) * ((nout + bno - 1) / bno);
 }
 
-// Fitted to measured launches of the 128 x 80 tiles (M = 192..4096, K =
-// 896..18944; 13 % rms): 5.4 us per round of workgroups and 1.32 us per
-// K-tile of a wave, 12 % more per further round (up to 6) as the clock drops
-// under the load.
+// Fitted to 673 measured launches of the 128 x 80 tiles (drawn shapes, M =
+// 150..4096, K = 512..18944, all epilogues; 6 % rms): a round of workgroups
+// costs 6 us and 1.2 us per K-tile of a wave, 5 % more per further round (up
+// to 6) as the clock drops under the load.  The epilogues work element by
+// element, ~10 us a round, and so do the stores of rows that are not 16-byte
+// aligned, 4 us.  (Without those two terms the estimate was up to 2.5 times
+// too low: M = 1091, K = N = 3072 with the residual stayed here at 64 us, 43 in
+// the many-row GEMM.)
 double gemm16_estimate(const LinearArgs& a, int cus) {
   const double r = (double)gemm16_workgroups(a) / cus;
-  const double per = 5.4 + a.K / 256.0 * (1.32 + 0.116 * std::max(0.0, std::min(r, 6.0) - 1.0));
-  return 4.3 + (r < 3.0 ? std::ceil(r) : r + 0.4) * per;
+  const double epi = a.epi == EPI_NONE ? 0.0 : a.epi == EPI_BIAS_SILU ? 11.79 : a.epi == EPI_RESIDUAL ? 9.80 : 9.11;
+  const double per = 5.81 + epi + (a.ldc % 8 ? 4.10 : 0.0) + a.K / 256.0 * (1.192 + 0.0663 * std::max(0.0, std::min(r, 6.0) - 1.0));
+  return 2.99 + (r < 3.0 ? std::ceil(r) : r + 0.4) * per;
 }
 
 hipError_t gemm16_launch(const LinearArgs& a, hipStream_t s, uint64_t* trace) {

@@ -634,46 +634,56 @@ namespace {
 // which must stay zero
 constexpr size_t kCntBytesN = 65536;
 
-// Launch-time model (microseconds), fitted to 774 (256-row tiles) and 1056
-// (128-row tiles) measured launches (M = 32..4096, K = 896..18944, N =
-// 896..37888, int4 and int8, 1-16 K parts, 5 % rms) and refitted with 1700
-// launches of drawn shapes (K = 512..18944, N = 512..37888, all group sizes and
-// epilogues), where it is 8 % off with K parts; without them 128- and 256-row
-// tiles take a quarter longer than it says, on shapes where the other kernels
-// are further off still.
-//  * 256 rows: one workgroup per CU.  A K-tile takes 1.22 us, and up to 1.70
-//    us when all CUs run (the clock drops under the load).
-//  * 128 rows: two workgroups fit a CU; a K-tile takes 0.77-1.05 us alone,
-//    2.02 us in each of two.
-//  * 64 rows: two workgroups fit a CU; a K-tile takes 0.70 us alone, 1.07 us in
-//    each of two (int8 0.10 and 0.30 more), and the bytes of scales, outputs
-//    and residual count (2536 launches, M = 17..512, 8 % rms).
-//  * K parts: their sums are written and read once, 0.14-0.22 us per MB, and a
-//    thread adds all parts of its 8 columns, 0.1 us a part, or 0.5 with SwiGLU
+// Launch-time model (microseconds), per tile height, fitted to 21300 measured
+// launches of 6000 drawn shapes (M = 17..4096, up to 640 with 64 rows; K =
+// 512..18944, N = 512..37888, int4 and int8, all group sizes and epilogues, 1-64
+// K parts): 7 % rms with 64 and 128 rows, 8 % with 256.
+//  * 256 rows: one workgroup per CU.  A K-tile takes 1.20 us, and 1.35 when
+//    all CUs run (the clock drops under the load).
+//  * 128 and 64 rows: two workgroups fit a CU.  A K-tile takes 0.82-0.93 us
+//    (128 rows) or 0.71-0.80 (64) alone, 1.94 or 1.36 in each of two.
+//  * int8 takes 0.10-0.33 us more per K-tile: twice the weight loads, and
+//    with 64 and 128 rows half the ring depth.
+//  * K parts: their sums are written and read once, 0.2 us per MB, and a
+//    thread adds all parts of its 8 columns, 0.16 us a part, or 0.5 with SwiGLU
 //    (half the threads with twice the loads; where they are few, nothing hides
-//    the loads' latency: M = 107, K = 4864, N = 896 in 19 parts takes 22 us, 14
-//    without this term).
+//    the loads' latency).
+//  * The bytes of scales, outputs and residual; rows that are not 16-byte
+//    aligned are written, and a residual read, element by element.
+struct NFit {
+  double launch, round, tile, load, i8;        // tile: a K-tile in a full CU
+  double two, alone, alone_i8, alone_load;     // two workgroups per CU: a K-tile of the second, of one alone
+  double scale_mb, out_mb, bias_mb, resid_mb, silu_mb, odd_mb, odd_resid_mb;
+  double split, split_swi, part, part_swi, part_mb, split_i8;
+};
+constexpr NFit kFit64 = {9.38, -4.33, 1.359, 0.009, 0.327, 1.186, 0.713, 0.112, 0.122, 0.955, 0.044, 0.270, 0.413,
+                         0.466, 0.683, 0.579, 1.56, -0.88, 0.156, 0.402, 0.229, 0.16};
+constexpr NFit kFit128 = {11.88, -4.48, 1.940, 0.273, 0.254, 1.421, 0.820, 0.102, 0.140, 0.484, 0.194, 0.101, 0.312,
+                          0.410, 0.571, 0.678, 0.28, -0.71, 0.160, 0.372, 0.210, 0.10};
+constexpr NFit kFit256 = {9.78, 1.19, 1.206, 0.136, 0.103, 0.0, 0.0, 0.0, 0.0, 0.117, 0.383, 0.094, 0.454,
+                          0.445, 0.575, 0.709, -1.80, -0.02, 0.172, 0.317, 0.205, 0.76};
+
 double estimate(const LinearArgs& a, int mb, int64_t wgs, int KP, int ktp, double part_mb, int cus) {
-  const bool swi = a.epi == EPI_SWIGLU, i8 = a.fmt == FMT_INT8;
-  const double split = KP > 1 ? 1.0 : 0.0, sum = split * (swi ? 0.47 : 0.10) * KP;
+  const NFit& f = mb == 8 ? kFit256 : mb == 4 ? kFit128 : kFit64;
+  const bool swi = a.epi == EPI_SWIGLU;
+  const double i8 = a.fmt == FMT_INT8 ? 1.0 : 0.0;
+  const double out_mb = 2e-6 * a.M * (swi ? a.F : a.N);
+  double t = f.launch + f.scale_mb * 4e-6 * a.N * a.G + f.out_mb * out_mb;
   if (mb == 8) {
-    const double rounds = (double)wgs / cus;
-    const double whole = std::ceil(rounds);
-    const double tk = 1.22 + 0.48 * std::max(0.0, std::min(1.0, rounds) - 0.5) * 2.0;
-    return 11.3 + (whole <= 3 ? whole : rounds + 0.5) * (1.97 + ktp * tk) + split * 0.29 + 0.143 * part_mb + sum;
+    const double rounds = (double)wgs / cus, whole = std::ceil(rounds);
+    const double tk = f.tile + f.i8 * i8 + f.load * 2.0 * std::max(0.0, std::min(1.0, rounds) - 0.5);
+    t += (whole <= 3 ? whole : rounds + 0.5) * (f.round + ktp * tk);
+  } else {
+    const int64_t slots = 2 * (int64_t)cus, full = wgs / slots, rem = wgs - full * slots;
+    t += full * (f.round + ktp * (f.tile + f.i8 * i8));
+    if (rem > cus) t += f.round + ktp * (f.two + f.i8 * i8 + f.load * (double)(rem - cus) / cus);
+    else if (rem > 0) t += f.round + ktp * (f.alone + f.alone_i8 * i8) * (1.0 + f.alone_load * (double)rem / cus);
   }
-  const int64_t slots = 2 * (int64_t)cus;
-  const int64_t full = wgs / slots, rem = wgs - full * slots;
-  if (mb == 2) {
-    const double scale_mb = 4e-6 * a.N * a.G, out_mb = 2e-6 * a.M * (swi ? a.N / 2 : a.N);
-    return 5.12 + (full + (rem > cus ? 1 : 0)) * ktp * (i8 ? 1.372 : 1.068) +
-           (rem > 0 && rem <= cus ? ktp * (i8 ? 0.796 : 0.696) : 0.0) + 0.756 * scale_mb + 0.729 * out_mb +
-           (a.epi == EPI_RESIDUAL ? 1.05 * out_mb : 0.0) + split * (1.51 + (swi ? 0.509 : 0.133) * KP) + 0.222 * part_mb;
-  }
-  double t = 8.05 + full * (1.55 + ktp * 2.02);
-  if (rem > cus) t += 1.55 + ktp * (0.77 + 1.25 * (0.6 + 0.4 * (double)(rem - cus) / cus));
-  else if (rem > 0) t += 1.55 + ktp * 0.77 * (1.0 + 0.36 * (double)rem / cus);
-  return t + split * (swi ? -0.62 : 0.45) + 0.19 * part_mb + sum;
+  if (a.epi == EPI_RESIDUAL) t += (f.resid_mb + (a.ldr % 8 ? f.odd_resid_mb : 0.0)) * out_mb;
+  if (epi_needs_bias(a.epi)) t += (f.bias_mb + (a.epi == EPI_BIAS_SILU ? f.silu_mb : 0.0)) * out_mb;
+  if (a.ldc % 8) t += f.odd_mb * out_mb;
+  if (KP > 1) t += f.split + f.split_i8 * i8 + f.part_mb * part_mb + f.part * KP + (swi ? f.split_swi + f.part_swi * KP : 0.0);
+  return t;
 }
 
 }  // namespace
@@ -686,7 +696,7 @@ GemmnPlan gemmn_plan(const LinearArgs& a, int cus, bool allow_split, int mb, int
   const int KT = (a.K + 63) / 64;
   const int64_t ld = (int64_t)((F + 7) & ~7) * (swi ? 2 : 1);
   for (int m = 2; m <= 8; m *= 2) {
-    if (mb ? m != mb : m == 2 && a.M > 320) continue;   // (64 rows: not the fastest beyond, and not modelled)
+    if (mb ? m != mb : m == 2 && a.M > 640) continue;   // (64 rows: on 676 shapes from 321 to 640 the fastest height on 255; not measured beyond)
     const int64_t tiles = (int64_t)((a.M + 32 * m - 1) / (32 * m)) * ((F + (swi ? 127 : 255)) / (swi ? 128 : 256));
     for (int q = 1; q <= (m == 2 ? 64 : 16); ++q) {
       if (kp && q != kp) continue;

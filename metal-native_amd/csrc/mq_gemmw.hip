@@ -706,27 +706,43 @@ bool gemmw_supported(const LinearArgs& a, int cus) {
 
 size_t gemmw_ws_bytes(const LinearArgs& a, int cus, bool allow_split) { return plan(a, cus, allow_split).ws_bytes; }
 
-// Per format and tile shape, fitted to 1217 (int4) and 661 (int8) measured
-// launches of drawn shapes (M = 17..4096, K = 544..18944, N = 512..37888; 12 %
-// and 13 % rms; launch_us, which only ranks this kernel's own tilings, is
+// Per format and tile shape, fitted to 2497 (int4) and 1275 (int8) measured
+// launches of drawn shapes (M = 17..4096, K = 512..18944, N = 512..37888; 8 %
+// and 10 % rms; launch_us, which only ranks this kernel's own tilings, is
 // further off there): a round of workgroups costs a fixed time and its
-// per-wave K-tiles times the tile's own, a little more when the rounds are
-// full; a residual is read element by element.
-double gemmw_estimate(const LinearArgs& a, int cus, bool allow_split) {
+// per-wave K-tiles times the tile's own; the epilogues and the stores of
+// unaligned rows work element by element (with K parts only the last arriver
+// of a tile does); scales and zeros count by their bytes.
+double gemmw_estimate(const LinearArgs& a, int cus, bool allow_split, bool* has_parts) {
   const WPlan p = plan(a, cus, allow_split);
+  if (has_parts) *has_parts = p.ok && p.KP > 1;
   if (!p.ok) return 0.0;
-  const bool i4 = a.fmt == FMT_INT4;
-  // us per K-tile of a wave; the shapes that plan() takes: MB x NB = 1 x 2, 2 x 2, 2 x 3, 2 x 4, 2 x 6, 4 x 2, 4 x 3
-  static const double tile4[7] = {0.389, 0.662, 1.140, 1.818, 2.602, 1.225, 2.212};
-  static const double tile8[7] = {0.499, 0.623, 1.217, 1.553, 2.880, 1.281, 1.872};
-  const int shape = p.MB == 1 ? 0 : p.MB == 2 ? (p.NB == 6 ? 4 : p.NB - 1) : p.NB + 3;
+  struct Out {
+    double bias, silu, resid, odd, swiglu;   // us per block of a tile (swiglu: per tile)
+  };
+  struct Fit {
+    double round, tile[7];      // us per round, per K-tile of a wave: MB x NB = 1 x 2, 2 x 2, 2 x 3, 2 x 4, 2 x 6, 4 x 2, 4 x 3
+    double split[3], part[3];   // K parts, for MB = 1, 2, 4: once, per part and block
+    double scale_mb[3];
+    Out whole, parts;
+  };
+  static const Fit i4 = {5.45, {0.361, 0.653, 1.196, 1.377, 2.387, 1.283, 2.402}, {3.73, 3.73, 6.06}, {0.070, 0.070, 0.068},
+                         {1.33, 1.02, 0.26}, {0.109, 0.301, 0.633, 0.137, 1.56}, {0.019, 0.304, 1.142, -0.036, 2.31}};
+  static const Fit i8 = {5.80, {0.454, 0.688, 1.219, 1.961, 2.872, 1.334, 2.426}, {4.02, 4.02, 4.40}, {0.060, 0.060, 0.123},
+                         {1.36, 1.19, 0.84}, {0.156, 0.354, 0.708, 0.122, 1.80}, {0.033, 0.268, 1.191, 0.014, 1.88}};
+  const Fit& f = a.fmt == FMT_INT4 ? i4 : i8;
+  const Out& o = p.KP > 1 ? f.parts : f.whole;
+  const int shape = p.MB == 1 ? 0 : p.MB == 2 ? (p.NB == 6 ? 4 : p.NB - 1) : p.NB + 3, mi = p.MB >> 1;
   const double per = std::ceil(a.K / 64.0) / p.KP / 4.0, mn = (double)p.MB * p.NB;
-  const double r = (double)((int64_t)p.nbm * p.nbn * p.KP) / cus, r1 = r / p.KP;
-  auto rounds = [](double x) { return std::ceil(x) <= 3.0 ? std::ceil(x) : x + 0.5; };
-  const double tile = (i4 ? tile4 : tile8)[shape] + (i4 ? 0.0173 : 0.0237) * mn * std::min(1.0, std::max(0.0, r - 0.5));
-  return rounds(r) * ((i4 ? 6.84 : 7.25) + per * tile) +
-         (p.KP > 1 ? (i4 ? 2.18 : 2.44) + (i4 ? 0.175 : 0.153) * p.KP * mn : 0.0) +
-         (a.epi == EPI_RESIDUAL ? (i4 ? 0.623 : 0.675) * mn * rounds(r1) : 0.0);
+  const double r = (double)((int64_t)p.nbm * p.nbn * p.KP) / cus, whole = std::ceil(r);
+  const double rounds = whole <= 3.0 ? whole : r + 0.5;
+  const double epi = a.epi == EPI_RESIDUAL ? o.resid : a.epi == EPI_BIAS_SILU ? o.silu : epi_needs_bias(a.epi) ? o.bias : 0.0;
+  const double out = mn * (epi + (a.ldc % 8 ? o.odd : 0.0)) + (a.epi == EPI_SWIGLU ? o.swiglu : 0.0);
+  // 4 x 2 tiles: narrower ones than the blocks hold are the faster ones
+  const bool swi = a.epi == EPI_SWIGLU, narrow = p.BN < (swi ? 16 : 32) * p.NB;
+  const double width = p.MB != 4 || p.NB != 2 ? 1.0 : narrow ? (swi ? 0.92 : 0.98) : (swi ? 1.0 : 1.06);
+  return width * (rounds * (f.round + per * f.tile[shape]) +
+                  (p.KP > 1 ? f.split[mi] + f.part[mi] * p.KP * mn + out : rounds * out) + f.scale_mb[mi] * 4e-6 * a.N * a.G);
 }
 
 hipError_t gemmw_launch(const LinearArgs& a, int cus, void* ws, hipStream_t s, bool allow_split) {

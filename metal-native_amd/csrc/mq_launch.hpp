@@ -122,8 +122,9 @@ hipError_t rstream_launch(const LinearArgs& a, const RsPlan& p, hipStream_t s);
 // that every launch leaves at zero, then the partial sums).
 bool gemmw_supported(const LinearArgs& a, int num_cus);
 size_t gemmw_ws_bytes(const LinearArgs& a, int num_cus, bool allow_split);
-// estimated launch time (us) of the plan, 0 when there is none
-double gemmw_estimate(const LinearArgs& a, int num_cus, bool allow_split);
+// estimated launch time (us) of the plan, 0 when there is none; *has_parts:
+// whether it splits K
+double gemmw_estimate(const LinearArgs& a, int num_cus, bool allow_split, bool* has_parts);
 hipError_t gemmw_launch(const LinearArgs& a, int num_cus, void* ws, hipStream_t s, bool allow_split);
 
 // 128-row int4 GEMM (16x16x32 MFMA, one workgroup per 128 x 80 tile, no
@@ -135,7 +136,8 @@ double gemm16_estimate(const LinearArgs& a, int num_cus);   // launch time (us)
 hipError_t gemm16_launch(const LinearArgs& a, hipStream_t s, uint64_t* trace);
 
 // GEMM for many rows (32x32x16 MFMA, waves side by side along N, shared
-// activation tiles, no workspace): 32 * mb rows per tile, mb = 2, 4 or 8.
+// activation tiles): 32 * mb rows per tile, mb = 2, 4 or 8; a workspace only
+// where K is split.
 bool gemmn_supported(const LinearArgs& a);
 // K may be split over KP workgroups per tile, whose fp32 sums (ws_bytes, need
 // not be cleared) a second kernel adds up.

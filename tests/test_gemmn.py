@@ -218,11 +218,26 @@ def test_routing(mn, gpu, M, K, N, g, qt, epi, want):
     check(y.cpu().numpy(), acc, epi, b, r, want)
 
 
+@pytest.mark.parametrize("M,K,N,g,qt,epi", [          # us: the other kernel / this one
+    (1091, 3072, 3072, 128, "int4", "residual"),      # 63.6 / 42.8: its epilogue works element by element
+    (834, 3584, 4608, 64, "int8", "bias"),            # 69.0 / 52.6
+    (293, 896, 9728, 64, "int4", "residual"),         # 42.8 / 19.1
+    (19, 3584, 37888, 64, "int4", "residual"),        # 52.9 / 41.5
+    (67, 18944, 3584, 128, "int4", "bias"),           # 60.1 / 33.6
+])
+def test_routing_takes_the_faster_kernel(mn, gpu, M, K, N, g, qt, epi):
+    x, wp, s, z, g, acc = problem(M, K, N, g, qt, seed=M)
+    kw, b, r = epilogue_args(epi, M, N, gpu)
+    y = mn.dequant_matmul(dev(x, gpu), dev(wp, gpu), dev(s, gpu), dev(z, gpu), g, qt, **kw)
+    assert mn.last_path() == "gemmn", mn.last_path()
+    check(y.cpu().numpy(), acc, epi, b, r)
+
+
 @pytest.mark.parametrize("M,K,N,g,qt,epi", [   # us: the kernel it is left to / this one
     (1941, 1120, 1298, 32, "int8", None),      # 21.0 / 28.1
     (117, 3424, 23562, 3424, "int8", None),    # 44.2 / 53.7
-    (19, 2144, 25754, 32, "int4", "swiglu"),   # 26.6 / 35.1
-    (107, 4864, 896, 128, "int4", "swiglu"),   # 18.9 / 22.2: many K parts for few threads to add
+    (21, 2560, 23744, 64, "int8", None),       # 25.7 / 37.5
+    (93, 4864, 896, 128, "int4", "swiglu"),    # 15.9 / 19.1: many K parts for few threads to add
     (93, 2304, 21770, 64, "int4", None),       # 27.6 / 31.9
     (452, 2336, 4572, 32, "int4", None),       # 28.2 / 32.1
 ])
@@ -331,7 +346,7 @@ def test_threads_on_one_stream(mn, gpu):
     import threading
 
     shapes = [(300, 8192, 2048, 128, "gemmn"), (130, 8192, 1024, 128, "gemmn"), (8, 8192, 3072, 128, None),
-              (37, 18944, 512, 128, "gemmn")]
+              (200, 18944, 512, 128, "gemmn")]
     calls, want = [], []
     for i, (M, K, N, g, path) in enumerate(shapes):
         args = tuple(dev(a, gpu) for a in O.make_int4_problem(M, K, N, g, seed=60 + i)) + (g, "int4")
