@@ -220,9 +220,10 @@ MQ_API int mq_attention_decode_rope_f16(const void* qkv, const float* cos_table,
  * aligned (fp32 [heads][4][head_dim] partial outputs, then [heads][4] pairs of
  * running maximum and weight sum).  mq_attention_parts_dequant_matmul: C[N] =
  * half(attention output) . deq(W)^T, W int4 [N, heads * head_dim].  Both run
- * where mq_attention_parts_supported (one int4 row of at most 8192 columns;
- * caches of more than 256 positions at head_dim 128, 512 at 64: the split
- * gains nothing in shorter ones); otherwise they return 4 and the caller runs
+ * where mq_attention_parts_supported (int4, heads * head_dim at most 4096, or
+ * 6144 where a compute unit's share of the weights is more than 64 KiB; caches
+ * of more than 256 positions at head_dim 128, 512 at 64: the split gains
+ * nothing in shorter ones); otherwise they return 4 and the caller runs
  * mq_attention_decode_rope_f16 and mq_dequant_matmul. */
 MQ_API int64_t mq_attention_parts_size(int32_t heads, int32_t head_dim);
 MQ_API int mq_attention_parts_supported(int64_t N, int32_t heads, int32_t head_dim, int64_t max_len, int32_t group_size,

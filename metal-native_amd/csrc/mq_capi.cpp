@@ -240,7 +240,13 @@ int choose_path(const mq::LinearArgs& a, bool noalloc, bool allow_parts, mq::Gem
   // automatic choice: the row-block kernel up to M = 4; for M = 5..16 only
   // where the activations fit in LDS whole (its K parts measured slower than
   // the split-K GEMV at config 2, M = 8: 20.3 vs 18.2 us; whole, it is
-  // faster: config 4 at M = 8, 29.5 vs 40.3 us, at M = 16, 31.8 vs 45.4 us)
+  // faster: config 4 at M = 8, 29.5 vs 40.3 us, at M = 16, 31.8 vs 45.4 us).
+  // int4 against the register-streamed GEMV, K = 896..4096 (11 shapes): M = 5
+  // and 8 5-40 % faster but for N around 1000 (equal), e.g. K = 3584, N = 4608
+  // 7.4 vs 10.0 us; M = 9..16 the slower one where both take the shape, 10.2 vs
+  // 9.4 us there at M = 13, 9.3 vs 7.7 at N = 3584, 7.9 vs 5.6 at K = 896, N =
+  // 1152; for N = 9728 and more only this one does (K >= 3584), or the split-K
+  // GEMV is faster (K = 896: 5.2 vs 9.3 us)
   if (a.M <= 4 && short_rows(a) && decode_ok(a)) return PATH_DECODE;
   if (a.M <= 4 && rows_ok(a)) return PATH_ROWS;
   if (a.M <= 16) {

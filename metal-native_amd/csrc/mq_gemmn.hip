@@ -30,27 +30,22 @@
 //    four adjacent output columns of one row; the epilogue goes through a
 //    per-wave LDS stage, 32 rows at a time, to 16-byte stores.
 //
-// Dequantization without forming q - 8 first.  A nibble alone in an fp16
-// (the other bits zero) is the subnormal q * 2^-24, or q * 2^-20 four bits
-// up.  With s = (1 + m) 2^(e - 15) and S = (1 + m) 2^10,
-//   fma(q * 2^-20, S, -8 (1 + m) 2^-10) = RNE((q - 8) (1 + m) 2^-10),
-// which is RNE((q - 8) s) but for the power of two P = 2^(e - 5): the addend is
-// exact and the result normal, so its one rounding is that of the product.
-// Then fma(., P, -z) = RNE(RNE((q - 8) s) - z): the two roundings of the
-// reference, in 4 instead of 5 VALU ops per pair of weights (the low nibbles
-// with 2^-14 and 16 P in place of 2^-10 and P; int8 takes u = q + 128 as
-// u * 2^-24).  It holds for 1 <= e <= 16 (2^-14 <= |s| < 4); a wave that meets
-// another scale takes the direct form for those K-tiles.
+// Dequantization without forming q - 8 first, as fast_dq of mq_device.hpp (where
+// its rounding is shown) but in natural k order, 4 instead of 5 VALU ops per
+// pair of weights; int8 takes u = q + 128 as u * 2^-24.  It holds for scales of
+// 2^-14 <= |s| < 4; a wave that meets another one takes the direct form for
+// those K-tiles.
 //
 // What it measures (M = 4096, K = 3584, N = 37888, int4 g = 128 with SwiGLU):
 // 1.05 ms, 1058 TFLOP/s, against 2.51 ms for the 64-column tiles of
 // mq_gemmw.hip; plain fp16 weights in the vendor library: 0.90 ms.  With all
-// CUs running it is bound by the clock that the matrix cores leave under load
-// (1.3-1.7 GHz; the same loop with nothing but its MFMAs: 0.79 ms).  Taking
-// one thing out of the loop at 18 workgroups (1.28 us a K-tile, full clock):
-// dequant 1.24, activation loads 1.12, fragment reads 1.27, weight loads 1.21,
-// all four 1.05; spreading the activation loads over the k-steps took it to
-// 1.21.  256 rows by 64 columns per wave keep the dequant at two VALU ops per
+// CUs running the clock drops to 1.76 GHz and the matrix cores are busy 54 % of
+// its cycles (counters); the same loop with nothing but its MFMAs takes 0.79
+// ms, which is all of the cycles at 1.3 GHz.  Taking one thing out of the loop
+// at 18 workgroups (1.28 us a K-tile, full clock; variants, not kept): dequant
+// 1.24, activation loads 1.12, fragment reads 1.27, weight loads 1.21, all four
+// 1.05; spreading the activation loads over the k-steps took it to 1.21.
+// 256 rows by 64 columns per wave keep the dequant at two VALU ops per
 // MFMA and LDS reads at 5/8 of its rate.  128-row tiles (two workgroups per
 // CU) dequantize twice as often and are within 3 % at full load; they fill
 // the CUs where there are fewer rows.
@@ -359,8 +354,9 @@ gemmn_kernel(GNArgs p) {
   }
 
   // the wave's own loads of the tile that is read next have landed: those
-  // issued after them are two tiles' activations and, at least, two tiles'
-  // weights (in the prologue the weights of WD tiles)
+  // issued after them are two tiles' activations and at least two tiles'
+  // weights; at tiles 0 and 1 of a 2-deep weight ring one tile's weights and
+  // the eight scale and zero loads of tile 0 (NW = 4 of them are needed)
   auto tile_ready = [&]() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * ND + 2 * NW) : "memory");
     __builtin_amdgcn_s_barrier();

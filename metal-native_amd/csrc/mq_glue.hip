@@ -629,7 +629,7 @@ hipError_t attn_parts_launch(const void* qkv, const float* cos_t, const float* s
                              void* vc, float* parts, int H, int KVH, int D, int64_t L, float scale, hipStream_t s) {
   if (!attn_parts_supported(H, D, L)) return hipErrorInvalidValue;
   const int64_t steps = (L + 4096 / D - 1) / (4096 / D);   // of 32 (D = 128) or 64 positions
-  const int NW = (int)std::min<int64_t>(12, (steps + kAttnParts - 1) / kAttnParts);   // one wave per step up to 12, at least 2
+  const int NW = (int)std::min<int64_t>(12, (steps + kAttnParts - 1) / kAttnParts);   // one wave per step up to 12, at least 3
   const dim3 g(H, kAttnParts), b(64 * NW);
   if (D == 128)
     hipLaunchKernelGGL((attn_head_d_kernel<128, true>), g, b, 0, s, (const _Float16*)qkv, cos_t, sin_t, pos,
