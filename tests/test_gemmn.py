@@ -224,6 +224,9 @@ def test_routing(mn, gpu, M, K, N, g, qt, epi, want):
     (293, 896, 9728, 64, "int4", "residual"),         # 42.8 / 19.1
     (19, 3584, 37888, 64, "int4", "residual"),        # 52.9 / 41.5
     (67, 18944, 3584, 128, "int4", "bias"),           # 60.1 / 33.6
+    (440, 832, 18390, 32, "int4", "residual"),        # 100.7 / 39.1: 64-row tiles, rows that are not 16-byte aligned
+    (589, 928, 5778, 32, "int8", "residual"),         # 45.6 / 30.0
+    (640, 896, 4870, 64, "int4", "swiglu"),           # the last M of 64-row tiles, the last columns past a tile
 ])
 def test_routing_takes_the_faster_kernel(mn, gpu, M, K, N, g, qt, epi):
     x, wp, s, z, g, acc = problem(M, K, N, g, qt, seed=M)
